@@ -13,7 +13,7 @@ import threading
 from pathlib import Path
 
 LIB_PATH = Path(__file__).resolve().parent / "_build" / "libdabsn_hip.so"
-ABI_VERSION = 18
+ABI_VERSION = 19
 
 _lock = threading.Lock()
 _lib = None
@@ -158,6 +158,11 @@ _SIGNATURES = {
     "dabsn_hip_means_glue": ([i64, i64, i64, vp, i64, PTR8, i32, vp, vp, vp, vp], i32),
     "dabsn_hip_ce_fwd": ([i32, i64, i64, vp, i64, vp, i64, vp, vp, vp, vp], i32),
     "dabsn_hip_ce_bwd": ([i32, i64, i64, vp, i64, vp, i64, vp, vp, vp, vp, vp], i32),
+    "dabsn_hip_ce_split_parts": ([i64], i64),
+    "dabsn_hip_ce_split": (
+        [i64, i64, vp, i64, vp, i64, vp, vp, vp, i64, i64, vp, vp, vp], i32),
+    "dabsn_hip_ce_bias": ([i64, i64, vp, i32, vp, vp], i32),
+    "dabsn_hip_ce_join": ([i64, vp, vp, vp], i32),
     "dabsn_hip_read3_decode": (
         [i32, i64, i64, i64, i64, vp, vp, i64, i64, vp, vp, vp, vp, vp, vp, vp, vp, vp, vp, PTR4,
          vp, vp, sz, vp],

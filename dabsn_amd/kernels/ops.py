@@ -989,6 +989,113 @@ def _ce_rows_backward_fake(logits, targets, ignore_index, lse, scale):
     return logits.new_empty(logits.shape, dtype=torch.float32)
 
 
+@torch.library.custom_op(_q("_ce_rows_word"), mutates_args=("word",), device_types="cuda")
+def ce_rows_word(logits: Tensor, targets: Tensor, ignore_index: int, word: Tensor,
+                 check: bool) -> tuple[Tensor, Tensor]:
+    """``ce_rows`` for one chunk of a longer row range: the kernel's error bits are OR-ed into
+    ``word`` (int32 [1], zero before the first chunk), which is read only with ``check``, so a
+    range of chunks waits for the device once."""
+    _require_cuda(logits)
+    x = _ce_logits(logits)
+    rows, V = (int(d) for d in x.shape)
+    lib = _lib.load()
+    t = targets.to(device=x.device, dtype=torch.int64).contiguous()
+    lse = torch.empty(rows, device=x.device, dtype=torch.float32)
+    nll = torch.empty_like(lse)
+    tk = KernelTimer.begin("ce_rows_fwd", x)
+    _lib.check(lib.dabsn_hip_ce_fwd(_code(x.dtype), rows, V, _p(x), int(x.stride(0)) if rows else V,
+                                    _p(t), int(ignore_index), _p(lse), _p(nll), _p(word),
+                                    _stream(x)), "cross entropy")
+    KernelTimer.end(tk)
+    if check:
+        _record_error_word(word.view(torch.uint8), "cross entropy", _TARGET_ERROR)
+    return lse, nll
+
+
+@ce_rows_word.register_fake
+def _ce_rows_word_fake(logits, targets, ignore_index, word, check):
+    rows = logits.shape[0]
+    return (logits.new_empty((rows,), dtype=torch.float32),
+            logits.new_empty((rows,), dtype=torch.float32))
+
+
+@torch.library.custom_op(_q("_linear_ce_backward_bf16"), mutates_args=(), device_types="cuda")
+def linear_ce_backward_bf16(hidden: Tensor, weight: Tensor, bias: Optional[Tensor],
+                            targets: Tensor, lse: Tensor, scale: Tensor, chunk_rows: int,
+                            ignore_index: int) -> tuple[Tensor, Tensor, Tensor]:
+    """(grad hidden [N, H], grad weight [V, H], grad bias [V] fp32; empty without a bias) of the
+    chunked readout loss for bf16 ``hidden`` and ``weight`` (reference loss.py:105-137, whose
+    gradient products run in fp32 on fp32 copies of both). Their values are bf16, so only the
+    fp32 gradient rows need more than bf16: the row kernel writes them as three bf16 planes
+    that hold all of their bits (``dabsn_hip_ce_split``) and the products are bf16 matrix
+    products with fp32 accumulation, over the planes of several chunks at once (as many as
+    fill the fp32 weight copy they replace), so that the fp32 weight gradient is read and
+    written once per group of chunks instead of once per chunk."""
+    _require_cuda(hidden)
+    lib = _lib.load()
+    N, H = (int(d) for d in hidden.shape)
+    V = int(weight.shape[0])
+    dev, f32 = hidden.device, torch.float32
+    hid = hidden.contiguous()
+    tgt = targets.to(device=dev, dtype=torch.int64).contiguous()
+    l = lse.to(f32).contiguous()
+    sc = scale.to(device=dev, dtype=f32).reshape(1).contiguous()
+    grad_hidden = torch.empty_like(hid)
+    grad_bias = torch.zeros(V if bias is not None else 0, device=dev, dtype=f32)
+    if N == 0:
+        return grad_hidden, torch.zeros_like(weight), grad_bias
+    # Planes of 6 rows V bytes against 4 V H of the fp32 weight copy.
+    chunk = max(1, min(int(chunk_rows), N))
+    group = min(N, chunk * max(1, (2 * H // 3) // chunk))
+    ldp = -(-V // 8) * 8
+    planes = torch.empty((3, group, ldp), device=dev, dtype=torch.bfloat16)
+    nparts = sum(lib.dabsn_hip_ce_split_parts(min(chunk, group - s)) for s in range(0, group, chunk))
+    part = torch.empty((nparts, V), device=dev, dtype=f32) if bias is not None else None
+    word = torch.zeros(1, device=dev, dtype=torch.int32)
+    grad_weight = None
+    for g0 in range(0, N, group):
+        g1 = min(N, g0 + group)
+        if g1 - g0 < group:  # the last, shorter group: planes of its own height
+            planes = planes.reshape(-1)[:3 * (g1 - g0) * ldp].reshape(3, g1 - g0, ldp)
+        used = 0
+        for s in range(g0, g1, chunk):
+            e = min(g1, s + chunk)
+            logits = _ce_logits(torch.nn.functional.linear(hid[s:e], weight, bias))
+            if logits.dtype != torch.bfloat16:
+                raise TypeError("cross entropy: the bf16 readout gave logits of "
+                                f"{logits.dtype}")
+            q = None if part is None else part[used:]
+            tk = KernelTimer.begin("ce_rows_bwd", logits)
+            _lib.check(lib.dabsn_hip_ce_split(
+                e - s, V, _p(logits), int(logits.stride(0)), _p(tgt[s:e]), int(ignore_index),
+                _p(l[s:e]), _p(sc), _p(planes[:, s - g0:]), (g1 - g0) * ldp, ldp, _p(q), _p(word),
+                _stream(logits)), "cross entropy backward")
+            KernelTimer.end(tk)
+            used += lib.dabsn_hip_ce_split_parts(e - s)
+        d = planes.view(3 * (g1 - g0), ldp)[:, :V]
+        rows = hid[g0:g1]
+        gh = torch.mm(d, weight, out_dtype=f32)
+        _lib.check(lib.dabsn_hip_ce_join((g1 - g0) * H, _p(gh), _p(grad_hidden[g0:g1]),
+                                         _stream(gh)), "cross entropy backward")
+        rows3 = torch.cat((rows, rows, rows))
+        if grad_weight is None:
+            grad_weight = torch.mm(d.t(), rows3, out_dtype=f32)
+        else:
+            torch.addmm(grad_weight, d.t(), rows3, out_dtype=f32, out=grad_weight)
+        if part is not None:
+            _lib.check(lib.dabsn_hip_ce_bias(used, V, _p(part), int(g0 > 0), _p(grad_bias),
+                                             _stream(part)), "cross entropy backward")
+    _record_error_word(word.view(torch.uint8), "cross entropy backward", _TARGET_ERROR)
+    return grad_hidden, grad_weight.to(weight.dtype), grad_bias
+
+
+@linear_ce_backward_bf16.register_fake
+def _linear_ce_backward_bf16_fake(hidden, weight, bias, targets, lse, scale, chunk_rows,
+                                  ignore_index):
+    return (torch.empty_like(hidden), torch.empty_like(weight),
+            hidden.new_empty((weight.shape[0] if bias is not None else 0,), dtype=torch.float32))
+
+
 # ---------------------------------------------------------------------------
 # Read output: proj + long_gain * long (read.py:435-438, 821-823)
 # ---------------------------------------------------------------------------
@@ -2232,6 +2339,8 @@ OPERATORS = (
     _q("_local_field_gather_backward"),
     _q("_ce_rows"),
     _q("_ce_rows_backward"),
+    _q("_ce_rows_word"),
+    _q("_linear_ce_backward_bf16"),
     _q("long_scan_fused"),
     _q("_long_scan_fused_backward"),
     _q("read_tape_stats"),

@@ -7,7 +7,9 @@ one readout GEMM (hipBLASLt through ``F.linear``), and one HIP row kernel
 logits once in their own dtype instead of an fp32 copy plus logsumexp / gather kernels.
 The backward recomputes each chunk's logits, forms (softmax - onehot) * scale in one row
 kernel (``ops.ce_rows_backward``, reusing the forward's logsumexp), and runs the two
-gradient GEMMs in fp32 as the reference does (loss.py:95-137).
+gradient GEMMs in fp32 as the reference does (loss.py:95-137); for bf16 readouts the fp32
+rows are split into three bf16 planes that hold all of their bits, and the GEMMs are bf16
+with fp32 accumulation (``ops.linear_ce_backward_bf16``).
 
 Same API, defaults and environment switch as the reference: ``DABSN_LOSS_CHUNK_SCORES``
 sets the element budget (default 2**24), ``off`` forces ``F.cross_entropy`` on the full
@@ -75,9 +77,15 @@ class ChunkedLinearCrossEntropy(torch.autograd.Function):
         acc = _accum_dtype(hidden.dtype)
         n = int(hidden.shape[0])
         lses, nlls = [], []
+        # On the device the chunks share one error word, read after the last of them.
+        word = (torch.zeros(1, device=hidden.device, dtype=torch.int32) if hidden.is_cuda
+                else None)
         for s, e in _spans(n, chunk_rows):
             logits = F.linear(hidden[s:e], weight, bias)
-            lse, nll = ops.ce_rows(logits, targets[s:e], ignore_index)
+            if word is None:
+                lse, nll = ops.ce_rows(logits, targets[s:e], ignore_index)
+            else:
+                lse, nll = ops.ce_rows_word(logits, targets[s:e], ignore_index, word, e == n)
             lses.append(lse)
             nlls.append(nll)
         lse, nll = _rows(lses, hidden), _rows(nlls, hidden)
@@ -93,6 +101,11 @@ class ChunkedLinearCrossEntropy(torch.autograd.Function):
         hidden, weight, bias, targets, denom, lse = ctx.saved_tensors
         acc = ctx.acc
         scale = (grad_output / denom).to(torch.float32).reshape(1)
+        if hidden.is_cuda and hidden.dtype == weight.dtype == torch.bfloat16 and (
+                bias is None or bias.dtype == torch.bfloat16):
+            gh, gw, gb = ops.linear_ce_backward_bf16(hidden, weight, bias, targets, lse, scale,
+                                                     ctx.chunk_rows, ctx.ignore_index)
+            return (gh, gw, None if bias is None else gb.to(bias.dtype), None, None, None)
         weight_acc = weight.to(acc)
         grad_hidden = torch.empty_like(hidden)
         grad_weight = torch.zeros_like(weight, dtype=acc)

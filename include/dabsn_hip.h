@@ -17,7 +17,7 @@
 #include <stddef.h>
 #include <stdint.h>
 
-#define DABSN_HIP_ABI_VERSION 18
+#define DABSN_HIP_ABI_VERSION 19
 
 /* Status codes returned by every entry point. */
 #define DABSN_OK 0
@@ -651,6 +651,19 @@ int dabsn_hip_ce_fwd(int dtype, int64_t rows, int64_t V, const void* logits, int
 int dabsn_hip_ce_bwd(int dtype, int64_t rows, int64_t V, const void* logits, int64_t ldl,
                      const int64_t* targets, int64_t ignore_index, const float* lse,
                      const float* scale, float* dlogits, uint32_t* err, hipStream_t stream);
+/* The backward of bf16 logits as three bf16 planes whose sum is the fp32 gradient, bit for
+ * bit (planes + k * plane, row stride ldp >= V, k = 0..2): the gradient products then run as
+ * bf16 matrix products. part (NULL or [dabsn_hip_ce_split_parts(rows)][V]) receives partial
+ * column sums of the fp32 gradient; dabsn_hip_ce_bias sums them in order into gbias [V] (added
+ * to it with `add`). dabsn_hip_ce_join: out (bf16 [n]) = the sum of three fp32 [n] arrays. */
+int64_t dabsn_hip_ce_split_parts(int64_t rows);
+int dabsn_hip_ce_split(int64_t rows, int64_t V, const void* logits, int64_t ldl,
+                       const int64_t* targets, int64_t ignore_index, const float* lse,
+                       const float* scale, void* planes, int64_t plane, int64_t ldp, float* part,
+                       uint32_t* err, hipStream_t stream);
+int dabsn_hip_ce_bias(int64_t nparts, int64_t V, const float* part, int add, float* gbias,
+                      hipStream_t stream);
+int dabsn_hip_ce_join(int64_t n, const float* planes, void* out, hipStream_t stream);
 
 #ifdef __cplusplus
 }

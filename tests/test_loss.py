@@ -135,3 +135,77 @@ def test_out_of_range_target_is_reported(cuda_device):
     x = torch.randn(3, 10, device=cuda_device)
     with pytest.raises(RuntimeError, match="outside"):
         L.chunked_cross_entropy_from_logits(x, torch.tensor([1, 10, 2], device=cuda_device))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("rows,V", [(1, 1), (15, 7), (16, 8), (17, 2047), (33, 2048), (16, 2056),
+                                    (40, 257)])
+def test_split_gradient_planes_hold_the_fp32_gradient(cuda_device, rows, V):
+    """The three bf16 planes of the readout's gradient sum to the fp32 gradient bit for bit
+    (bf16 logits, ignored rows, an infinite logit's NaN row), and the bias partials to its
+    column sums: rows fp32 additions of terms below 1, so rows * 2^-24 each."""
+    from dabsn_amd import _lib
+    from dabsn_amd.kernels import ops
+
+    g = torch.Generator().manual_seed(rows * 10007 + V)
+    x = (torch.randn(rows, V, generator=g) * 4).to(torch.bfloat16)
+    if rows == 40:
+        x[3, 5] = float("inf")
+    t = torch.randint(0, V, (rows,), generator=g)
+    t[::5] = -100
+    x, t = x.to(cuda_device), t.to(cuda_device)
+    lse, _ = ops.ce_rows(x, t, -100)
+    scale = torch.tensor([0.37], device=cuda_device)
+    want = ops.ce_rows_backward(x, t, -100, lse, scale)
+    lib, ldp = _lib.load(), -(-V // 8) * 8
+    planes = torch.zeros(3, rows, ldp, device=cuda_device, dtype=torch.bfloat16)
+    part = torch.empty(lib.dabsn_hip_ce_split_parts(rows), V, device=cuda_device)
+    word = torch.zeros(1, device=cuda_device, dtype=torch.int32)
+    p = lambda v: v.data_ptr()  # noqa: E731
+    assert lib.dabsn_hip_ce_split(rows, V, p(x), V, p(t), -100, p(lse), p(scale), p(planes),
+                                  rows * ldp, ldp, p(part), p(word), None) == 0
+    torch.cuda.synchronize()
+    d = planes.double().sum(0)[:, :V]
+    assert torch.equal(torch.nan_to_num(d, 7.0, 8.0, 9.0),
+                       torch.nan_to_num(want.double(), 7.0, 8.0, 9.0))
+    if rows != 40:  # there the NaN row leaves no finite column sum
+        err = (part.double().sum(0) - want.double().sum(0)).abs().max()
+        assert float(err) <= rows * 2.0 ** -24
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("N,V,H,budget,bias", [(1, 5, 3, None, True), (70, 33, 48, 16 * 33, True),
+                                               (64, 129, 96, 16 * 129, False),
+                                               (300, 1000, 200, 40 * 1000, True),
+                                               (513, 4099, 73, 1 << 18, True)])
+def test_bf16_readout_gradients_match_fp64(cuda_device, N, V, H, budget, bias):
+    """One chunk, several chunks in a group, several groups with a shorter last one, odd
+    vocabularies and widths: gradients against fp64 on the same bf16 values. The logits are
+    rounded to bf16 (2^-9 of values up to about 5 standard deviations, an error of some
+    1e-2 in a softmax weight, random over a row's terms) and the gradients once more
+    (2^-9), so 1e-2 in the norm."""
+    h, w, b, t = _case(N + V, 1, N, H, V, bias=bias, dtype=torch.bfloat16)
+    t[:, ::7] = -100
+    leaves = [None if x is None else x.to(cuda_device).requires_grad_(True) for x in (h, w, b)]
+    loss = L.chunked_linear_cross_entropy(*leaves, t.to(cuda_device), chunk_budget=budget)
+    loss.backward()
+    ref_loss, ref = _naive(h, w, b, t)
+    if t.ne(-100).any():
+        assert abs(float(loss.detach()) - float(ref_loss)) <= 1e-2 * abs(float(ref_loss))
+        for a, r in zip(leaves, ref):
+            assert (a is None) == (r is None)
+            if a is not None:
+                assert a.grad.dtype == torch.bfloat16
+                err = (a.grad.double().cpu() - r).norm() / r.norm()
+                assert float(err) <= 1e-2
+    else:  # every row ignored
+        assert all(a is None or float(a.grad.float().abs().max()) == 0 for a in leaves)
+
+
+@pytest.mark.gpu
+def test_bf16_readout_reports_a_bad_target_in_any_chunk(cuda_device):
+    h, w, b, t = _case(9, 1, 40, 16, 30, dtype=torch.bfloat16)
+    t[0, 3] = 30
+    with pytest.raises(RuntimeError, match="outside"):
+        L.chunked_linear_cross_entropy(h.to(cuda_device), w.to(cuda_device), b.to(cuda_device),
+                                       t.to(cuda_device), chunk_budget=8 * 30)
