@@ -149,6 +149,8 @@ _SIGNATURES = {
     "dabsn_hip_read_dense_bwd": (
         [i64] * 4 + [vp] + [vp] * 8 + [vp] * 4 + [vp] + [vp] * 9 + [vp, sz, vp], i32),
     "dabsn_hip_permanent_scan_fwd": ([i64, i64, i64, vp, vp, vp, vp, vp], i32),
+    "dabsn_hip_permanent_scan_fwd_workspace_bytes": ([i64, i64, i64], sz),
+    "dabsn_hip_permanent_scan_fwd_ws": ([i64, i64, i64, vp, vp, vp, vp, vp, sz, vp], i32),
     "dabsn_hip_permanent_scan_workspace_bytes": ([i64, i64, i64], sz),
     "dabsn_hip_permanent_scan_bwd": ([i64, i64, i64, vp, vp, vp, vp, vp, vp, vp, vp, sz, vp], i32),
     "dabsn_hip_local_field_workspace_bytes": ([i64, i64, i64, i32], sz),

@@ -648,9 +648,11 @@ def permanent_delta_scan(k: Tensor, v: Tensor, beta: Tensor) -> Tensor:
     lib = _lib.load()
     kf, vf, bf = (x.float().contiguous() for x in (k, v, beta))
     out = torch.empty((B, T, H), device=k.device, dtype=torch.float32)
+    nbytes = lib.dabsn_hip_permanent_scan_fwd_workspace_bytes(B, T, H)
+    ws = torch.empty(max(nbytes, 4), dtype=torch.uint8, device=k.device)
     tk = KernelTimer.begin("permanent_scan_fwd", k)
-    _lib.check(lib.dabsn_hip_permanent_scan_fwd(B, T, H, _p(kf), _p(vf), _p(bf), _p(out),
-                                                _stream(k)), "permanent scan")
+    _lib.check(lib.dabsn_hip_permanent_scan_fwd_ws(B, T, H, _p(kf), _p(vf), _p(bf), _p(out),
+                                                   _p(ws), nbytes, _stream(k)), "permanent scan")
     KernelTimer.end(tk)
     return out.to(v.dtype)
 

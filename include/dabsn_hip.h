@@ -604,13 +604,20 @@ int dabsn_hip_read_dense_bwd(int64_t B, int64_t T, int64_t N, int64_t H, const f
  * key, value [B,T,H], beta [B,T], fp32 (the op converts other dtypes). Per batch row a
  * state S [H,H] starts at zero; out_t = S k_t, then S += beta_t (v_t - out_t) k_t^T.
  * H <= 2048. Backward: dkey, dvalue [B,T,H], dbeta [B,T] fp32 from grad_out [B,T,H]; it
- * recomputes the per-row states into the workspace, keeping every 8th one and the last
- * (dabsn_hip_permanent_scan_workspace_bytes(): 4 B (ceil(T/8)+1) H^2 bytes plus r_t and
- * partial sums), and rebuilds the states in between by undoing each step's update; the
- * reference's reverse pass keeps all T states. Results are deterministic. */
+ * recomputes the states into the workspace (dabsn_hip_permanent_scan_workspace_bytes()):
+ * those entering each chunk of 16 steps up to H = 512, every 8th one and the last beyond,
+ * with the states in between rebuilt by undoing each step's update; the reference's reverse
+ * pass keeps all T states. Results are deterministic. */
 int dabsn_hip_permanent_scan_fwd(int64_t B, int64_t T, int64_t H, const float* key,
                                  const float* value, const float* beta, float* out,
                                  hipStream_t stream);
+/* The same scan in chunks of 16 steps as fp32 matrix products (H <= 512; wider states walk
+ * step by step as above), with a workspace of
+ * dabsn_hip_permanent_scan_fwd_workspace_bytes() for the chunks' key products. */
+size_t dabsn_hip_permanent_scan_fwd_workspace_bytes(int64_t B, int64_t T, int64_t H);
+int dabsn_hip_permanent_scan_fwd_ws(int64_t B, int64_t T, int64_t H, const float* key,
+                                    const float* value, const float* beta, float* out,
+                                    void* workspace, size_t workspace_bytes, hipStream_t stream);
 size_t dabsn_hip_permanent_scan_workspace_bytes(int64_t B, int64_t T, int64_t H);
 int dabsn_hip_permanent_scan_bwd(int64_t B, int64_t T, int64_t H, const float* key,
                                  const float* value, const float* beta, const float* grad_out,

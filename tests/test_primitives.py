@@ -90,6 +90,50 @@ def test_permanent_scan_matches_oracle(cuda_device, B, T, H, unit):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("B,T,H", [(1, 2, 1), (2, 15, 15), (1, 16, 17), (3, 17, 64), (1, 31, 66),
+                                   (2, 48, 129), (1, 33, 255), (1, 65, 256), (1, 35, 511),
+                                   (1, 20, 512), (1, 18, 513)])
+def test_permanent_scan_chunk_and_tile_edges(cuda_device, B, T, H):
+    """Chunks of 16 steps, 16 value rows a workgroup and 64-column tiles up to H = 512, the
+    per-step walk beyond: one short, exact and one over each. fp32, against fp64: a value is
+    a sum over at most H + T fp32 products of values of order 1, so 1e-5 in the norm."""
+    from oracle import autograd_ref
+
+    k, v, beta, up = _permanent_case(90 + H + T, B, T, H)
+    leaves = [x.double().requires_grad_(True) for x in (k, v, beta)]
+    want = autograd_ref.permanent_loop(*leaves)
+    wgrads = torch.autograd.grad((want * up.double()).sum(), leaves)
+    mine = [x.to(cuda_device).requires_grad_(True) for x in (k, v, beta)]
+    out = ops.permanent_delta_scan(*mine)
+    grads = torch.autograd.grad((out * up.to(cuda_device)).sum(), mine)
+    for got, w in zip((out, *grads), (want, *wgrads)):
+        err = (got.detach().cpu().double() - w).norm()
+        assert float(err) <= 1e-5 * max(float(w.norm()), 1e-30)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("H", [40, 200])
+def test_permanent_scan_keeps_a_bad_step_out_of_the_steps_before_it(cuda_device, H):
+    """A NaN value row and an infinite key at one step, inside a chunk: the outputs before it
+    are those of the finite scan bit for bit; a NaN upstream gradient leaves dv after it so."""
+    k, v, beta, up = (x.to(cuda_device) for x in _permanent_case(7, 2, 40, H))
+    clean = ops.permanent_delta_scan(k, v, beta)
+    bad_v, bad_k = v.clone(), k.clone()
+    bad_v[:, 21, 3] = float("nan")
+    bad_k[:, 21, 5] = float("inf")
+    for kk, vv in ((k, bad_v), (bad_k, v)):
+        out = ops.permanent_delta_scan(kk, vv, beta)
+        assert torch.equal(out[:, :21], clean[:, :21])
+        assert not torch.isfinite(out[:, 22:]).all()
+    dv = ops.permanent_delta_scan_backward(k, v, beta, up)[1]
+    bad_up = up.clone()
+    bad_up[:, 21, 3] = float("nan")
+    bad = ops.permanent_delta_scan_backward(k, v, beta, bad_up)[1]
+    assert torch.equal(bad[:, 21:], dv[:, 21:])
+    assert torch.isnan(bad[:, :21, 3]).all()
+
+
+@pytest.mark.gpu
 def test_permanent_scan_backward_is_deterministic(cuda_device):
     k, v, beta, up = (x.to(cuda_device) for x in _permanent_case(3, 2, 24, 200))
     first = ops.permanent_delta_scan_backward(k, v, beta, up)
