@@ -13,16 +13,21 @@
 // chained recurrences: E_t = er E + (1-er) w (constant coefficient), R_t = rd R +
 // (1-rd)(1 - pe_t) with pe_t = tanh|w_t - E_{t-1}| (constant coefficient, input known once
 // E is), and L_t = eff_t L + (1 - eff_t) sal_t w_t (coefficient eff_t known once R is).
-// T is cut into chunks of CK steps. For each recurrence in turn, a chunk-parallel pass
-// computes every chunk's end value from a zero start (plus the product of eff_t for L),
-// and a per-channel pass over the chunks turns those into the true chunk-start values
-// (the checkpoint, [B][nseg][3][H] fp32, kept for the backward). A last chunk pass writes
-// the output. The backward composes each chunk's affine map of the three adjoints (see the
-// backward kernels below) and carries the maps across chunks in one per-channel pass; both
-// of its chunk passes replay the forward recurrence over their chunk from the checkpoint
-// (the same step function as the forward, so the replayed states are the forward's bits)
-// instead of reading per-step states, which would be 12 bytes per (row, step, unit) written
-// once and read twice.
+// T is cut into chunks of CK steps. A workgroup owns 64 channels of one batch row (16 where
+// channels are few); each of its waves holds one chunk's inputs in registers (four chunks of 16
+// channels), and the workgroup walks T in blocks of as many chunks as its waves hold. For each recurrence in turn every wave computes its chunk's end value from a zero
+// start (and the product of eff_t for L), one barrier shares the ends through LDS, and every
+// wave folds the chunks before its own into its true start. So the inputs are read once and
+// tanh is evaluated once per step, between one read and one write of memory (the earlier form
+// ran a kernel per recurrence: four reads of w, three tanh). The chunk starts are the
+// checkpoint, [B][nseg][3][H] fp32, kept for the backward, which replays each chunk's forward
+// from it with the same step function (the same bits) and then carries the three adjoints
+// backward the same way: gL, then gR, then gE.
+//
+// Bound by memory and, nearly as much, by the vector ALU (a step is about 56 instructions
+// forward and 91 backward): see the figures at the launchers.
+#include <type_traits>
+
 #include "../../include/dabsn_hip.h"
 #include "capi.hpp"
 #include "common.hpp"
@@ -107,20 +112,38 @@ struct Logits {
   const float* p[4];
 };
 
-// One step of the three recurrences from the states entering it (L, E, R), in the step
-// order of long.py:492-579: pe = tanh|w - E|, then E, R, the retention eff and L advance.
-// Every pass that walks the recurrence (forward, and the backward's replays) calls this,
-// so the states a replay produces are bit-identical to the forward's.
-__device__ __forceinline__ void advance(const Coef& k, float wt, float pt, float& L, float& Ev,
-                                        float& R, float& pe, float& eff) {
-  pe = tanhf(fabsf(wt - Ev));
-  Ev = k.er * Ev + (1.0f - k.er) * wt;
-  R = k.rd * R + (1.0f - k.rd) * (1.0f - pe);
-  const float sal = pt * pe;
-  eff = k.ret + (1.0f - k.ret) * k.rs * R;
-  L = eff * L + (1.0f - eff) * (sal * wt);
+// tanh(y) for y >= 0 without a branch (the library's takes one per range, both in a wave whose
+// lanes disagree, and the unrolled steps around it cannot be interleaved). Below 0.625 the odd
+// polynomial y + y^3 q(y^2), q fitted to (tanh y - y) / y^3 by minimax least squares (relative
+// error 4.4e-9 before rounding); above, 1 - 2 / (exp(2y) + 1). At most 2 ulp, on average 2.4e-8
+// relative. NaN stays NaN, infinity gives 1.
+__device__ __forceinline__ float tanh_abs(float y) {
+  const float z = y * y;
+  float q = fmaf(-0.0057049826718866825f, z, 0.02063908241689205f);
+  q = fmaf(q, z, -0.05373971536755562f);
+  q = fmaf(q, z, 0.13331441581249237f);
+  q = fmaf(q, z, -0.3333328068256378f);
+  const float small = fmaf(y * z, q, y);
+  const float e = __builtin_amdgcn_exp2f(y * 2.8853900817779268f);  // exp(2y)
+  const float large = fmaf(-2.0f, __builtin_amdgcn_rcpf(e + 1.0f), 1.0f);
+  return y < 0.625f ? small : large;
 }
 
+// The pieces of one step of the three recurrences (long.py:492-579) from the states entering
+// it: pe = tanh|w - E|, then E, R, the retention eff and L advance. Every pass that walks the
+// recurrence (forward, and the backward's replays) calls these, so the states a replay
+// produces are bit-identical to the forward's. L advances as eff L + y, y = (1 - eff) x: not as
+// x + eff (L - x), two instructions shorter, whose difference rounds at the size of x, which
+// is well above that of its mean L.
+__device__ __forceinline__ float step_E(const Coef& k, float Ev, float wt) {
+  return fmaf(k.er, Ev, (1.0f - k.er) * wt);
+}
+__device__ __forceinline__ float step_R(const Coef& k, float R, float pe) {
+  return fmaf(k.rd, R, (1.0f - k.rd) * (1.0f - pe));
+}
+__device__ __forceinline__ float retention(const Coef& k, float R) {
+  return fmaf((1.0f - k.ret) * k.rs, R, k.ret);
+}
 // er^n for n <= CK by repeated multiplication (fixed order).
 __device__ __forceinline__ float powi(float x, int n) {
   float r = 1.0f;
@@ -128,86 +151,218 @@ __device__ __forceinline__ float powi(float x, int n) {
   return r;
 }
 
-struct ChunkIdx {
-  int64_t ch;       // b * H + h
-  int b, h, k, t0, len, nseg;
-  size_t base;      // offset of (b, 0, h) in [B, T, H]
-  size_t ibase;     // offset of (b, 0, h) in the inputs w, p (batch rows ldx apart)
-  size_t cbase;     // offset of (b, k, 0, h) in the checkpoint [B][nseg][3][H]
-};
+// A wave holds G chunks of 64 / G channels of one batch row; a workgroup of NW waves walks T in
+// blocks of NW G chunks.
+constexpr int LANES = 64;
 
-__device__ __forceinline__ bool chunk_idx(int B, int T, int H, int64_t ldx, ChunkIdx& c) {
-  c.ch = static_cast<int64_t>(blockIdx.x) * NT + threadIdx.x;
-  if (c.ch >= static_cast<int64_t>(B) * H) return false;
-  c.b = static_cast<int>(c.ch / H);
-  c.h = static_cast<int>(c.ch % H);
-  c.k = blockIdx.y;
-  c.t0 = c.k * CK;
-  c.len = min(CK, T - c.t0);
-  c.nseg = (T + CK - 1) / CK;
-  c.base = static_cast<size_t>(c.b) * T * H + c.h;
-  c.ibase = static_cast<size_t>(c.b) * ldx + c.h;
-  c.cbase = (static_cast<size_t>(c.b) * c.nseg + c.k) * 3 * H + c.h;
-  return true;
+// Folds the chunk ends `loc` (from a zero start, [chunk][channel]) of a block of `live` chunks
+// into the state x entering the block: returns the state entering chunk `idx`, x becomes the
+// state leaving the block. A chunk multiplies its entering state by prod[chunk], or by `power`
+// (coef^steps, one value for all). REV: the chunks in reverse (adjoints).
+template <int NC, int LC, bool REV>
+__device__ __forceinline__ float enter(float& x, const float (*loc)[LC], const float (*prod)[LC],
+                                       float power, int idx, int lc, int live) {
+  float mine = x;
+#pragma unroll
+  for (int q = 0; q < NC; ++q) {
+    const int j = REV ? NC - 1 - q : q;
+    mine = j == idx ? x : mine;
+    if (j < live) x = fmaf(prod ? prod[j][lc] : power, x, loc[j][lc]);
+  }
+  return mine;
 }
 
-// Forward chunk pass. PHASE 0: E from 0 -> loc0 = E end. PHASE 1: E from its true start,
-// R from 0 -> loc0 = R end. PHASE 2: E, R from true starts, L from 0 -> loc0 = L end,
-// loc1 = prod eff. PHASE 3: all from true starts (the checkpoint) -> out.
-template <typename E, int PHASE>
-__global__ void __launch_bounds__(NT) long_fwd_chunk(int B, int T, int H, int64_t ldx,
-                                                     const E* w, const E* p, Logits lg,
-                                                     const float* ckpt, float* loc0,
-                                                     float* loc1, E* out) {
-  ChunkIdx c;
-  if (!chunk_idx(B, T, H, ldx, c)) return;
-  const Coef k = load_coef(lg.p);
-  float wv[CK], pv[CK];
-#pragma unroll
-  for (int i = 0; i < CK; ++i) {
-    // Clamped, unconditional loads so all CK requests are in flight at once (steps past
-    // the chunk end are never used).
-    const size_t o = c.ibase + static_cast<size_t>(c.t0 + min(i, c.len - 1)) * H;
-    wv[i] = ld(w, o);
-    if (PHASE >= 2) pv[i] = ld(p, o);
+// Hides a value's history from the compiler, which otherwise keeps what one walk derives from it
+// (conversions, products with a constant) in registers for the next walk: 32 values each time.
+template <typename V>
+__device__ __forceinline__ void opaque(V& v) {
+  asm volatile("" : "+v"(v));
+}
+
+// The rows of one chunk of a [.., T, H] tensor as a wave reads and writes them: row i of the
+// chunk, this lane's channel. As buffer accesses the row is a scalar offset and the lane a
+// 32-bit one that stays put, so no address takes vector registers or instructions. Lanes past H
+// get an offset past any chunk (reads give zero, writes are dropped), and so do the rows past
+// `rows`. `first`: the lane's first row (its chunk's, where a wave holds several). Offsets are
+// 32 bits: rows of 2^24 elements and more use plain pointers.
+template <typename E, bool BIG>
+struct Rows {
+  __amdgpu_buffer_rsrc_t r;
+  uint32_t voff, row;
+  __device__ __forceinline__ Rows(E* p, int H, int h, int rows, int first = 0)
+      : row(static_cast<uint32_t>(H) * sizeof(E)) {
+    const uint64_t a = reinterpret_cast<uint64_t>(p);
+    const uint64_t u = static_cast<uint64_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(a))) & 0xffffffffu;
+    const uint64_t v = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(a >> 32)));
+    r = make_rsrc(reinterpret_cast<const void*>(u | v << 32), rows * row);
+    voff = h < H && first < rows ? static_cast<uint32_t>(h) * sizeof(E) + first * row : 0x80000000u;
   }
-  float Ev = PHASE >= 1 ? ckpt[c.cbase + H] : 0.0f;
-  float R = PHASE >= 2 ? ckpt[c.cbase + 2 * H] : 0.0f;
-  float L = PHASE >= 3 ? ckpt[c.cbase] : 0.0f;
-  float prod = 1.0f;
-#pragma unroll
-  for (int i = 0; i < CK; ++i) {
-    if (i < c.len) {
-      if (PHASE == 3) {
-        float pe, eff;
-        advance(k, wv[i], pv[i], L, Ev, R, pe, eff);
-        st(out, c.base + static_cast<size_t>(c.t0 + i) * H, L);
-        continue;
-      }
-      const float pe = PHASE >= 1 ? tanhf(fabsf(wv[i] - Ev)) : 0.0f;
-      Ev = k.er * Ev + (1.0f - k.er) * wv[i];
-      if (PHASE >= 1) R = k.rd * R + (1.0f - k.rd) * (1.0f - pe);
-      if (PHASE >= 2) {
-        const float sal = pv[i] * pe;
-        const float eff = k.ret + (1.0f - k.ret) * k.rs * R;
-        L = eff * L + (1.0f - eff) * (sal * wv[i]);
-        prod *= eff;
-      }
+  __device__ __forceinline__ E load(int i) const {
+    if constexpr (sizeof(E) == 2) {
+      return __builtin_amdgcn_raw_buffer_load_b16(r, voff, i * row, 0);
+    } else {
+      const uint32_t w = __builtin_amdgcn_raw_buffer_load_b32(r, voff, i * row, 0);
+      return __builtin_bit_cast(E, w);
     }
   }
-  const size_t li = static_cast<size_t>(c.k) * B * H + c.ch;
-  if (PHASE == 0) loc0[li] = Ev;
-  if (PHASE == 1) loc0[li] = R;
-  if (PHASE == 2) {
-    loc0[li] = L;
-    loc1[li] = prod;
+  __device__ __forceinline__ void store(int i, E v) const {
+    if constexpr (sizeof(E) == 2)
+      __builtin_amdgcn_raw_buffer_store_b16(v, r, voff, i * row, 0);
+    else
+      __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, v), r, voff, i * row, 0);
+  }
+};
+template <typename E>
+struct Rows<E, true> {
+  E* p;
+  size_t row;
+  bool ok;
+  __device__ __forceinline__ Rows(E* q, int H, int h, int rows, int = 0)
+      : p(q + min(h, H - 1)), row(static_cast<size_t>(H)), ok(rows > 0 && h < H) {}
+  __device__ __forceinline__ E load(int i) const { return p[i * row]; }
+  __device__ __forceinline__ void store(int i, E v) const {
+    if (ok) p[i * row] = v;
+  }
+};
+
+// Every 8th step, nothing moves across: steps interleave within a group, without all 32 of a
+// chunk in flight (and in registers) at once.
+__device__ __forceinline__ void fence(int i) {
+  if (i % 8 == 7) __builtin_amdgcn_sched_barrier(0);
+}
+
+// A wave of NW workgroup waves as a scalar, so the addresses of its chunk are scalar too.
+__device__ __forceinline__ int wave_id() {
+  return __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x) >> 6);
+}
+
+// Occupancy: the forward holds 2 values per step (at most 128 registers, 16 waves per CU).
+template <typename E, int NW, int G, bool BIG>
+__global__ void __launch_bounds__(NW* LANES, 4)
+    long_fwd_kernel(int T, int H, int64_t ldx, const E* __restrict__ w, const E* __restrict__ p,
+                    Logits lg, const float* __restrict__ L0, const float* __restrict__ E0,
+                    const float* __restrict__ R0, E* __restrict__ out, float* __restrict__ LF,
+                    float* __restrict__ EF, float* __restrict__ RF, float* __restrict__ ckpt) {
+  constexpr int NC = NW * G, LC = LANES / G;
+  __shared__ float se[NC][LC], sr[NC][LC], sl[NC][LC], sp[NC][LC];
+  const int lane = threadIdx.x & 63, wave = wave_id();
+  const int lc = lane % LC, sub = lane / LC, idx = wave * G + sub;
+  const int h = blockIdx.x * LC + lc, b = blockIdx.y;
+  const bool ok = h < H;
+  const int hc = ok ? h : H - 1;
+  const Coef k = load_coef(lg.p);
+  const float er_full = powi(k.er, CK), rd_full = powi(k.rd, CK);
+  const size_t ch = static_cast<size_t>(b) * H + hc;
+  float Lc = L0[ch], Ec = E0[ch], Rc = R0[ch];
+  E* wb = const_cast<E*>(w) + static_cast<size_t>(b) * ldx;
+  E* pb = const_cast<E*>(p) + static_cast<size_t>(b) * ldx;
+  E* ob = out + static_cast<size_t>(b) * T * H;
+  const int nseg = (T + CK - 1) / CK, nfull = T / CK, tail = T % CK;
+  auto keep = [&](int seg, float l, float e, float r) {
+    float* c = ckpt + (static_cast<size_t>(b) * nseg + seg) * 3 * H;
+    c[h] = l;
+    (c + H)[h] = e;
+    (c + 2 * static_cast<size_t>(H))[h] = r;
+  };
+  for (int k0 = 0; k0 < nfull; k0 += NC) {  // blocks of full chunks
+    const int live = min(NC, nfull - k0), seg = k0 + idx;
+    const bool mine = idx < live;
+    const int wlive = min(max(live - wave * G, 0), G);  // chunks of this wave
+    const size_t base = static_cast<size_t>(wlive > 0 ? k0 + wave * G : 0) * CK * H;
+    const Rows<E, BIG> wr(wb + base, H, h, wlive * CK, sub * CK),
+        pr(pb + base, H, h, wlive * CK, sub * CK), orow(ob + base, H, h, wlive * CK, sub * CK);
+    E wv[CK], pv[CK];
+#pragma unroll
+    for (int i = 0; i < CK; ++i) {
+      wv[i] = wr.load(i);
+      pv[i] = pr.load(i);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    float e = 0.0f;
+#pragma unroll
+    for (int i = 0; i < CK; ++i) {
+      e = step_E(k, e, to_f(wv[i]));
+      fence(i);
+    }
+#pragma unroll
+    for (int i = 0; i < CK; ++i) opaque(wv[i]);
+    se[idx][lc] = e;
+    __syncthreads();
+    const float Es = enter<NC, LC, false>(Ec, se, nullptr, er_full, idx, lc, live);
+    float pe[CK], x[CK];
+    float r = 0.0f;
+    e = Es;
+#pragma unroll
+    for (int i = 0; i < CK; ++i) {
+      const float wt = to_f(wv[i]);
+      pe[i] = tanh_abs(fabsf(wt - e));
+      x[i] = (to_f(pv[i]) * pe[i]) * wt;
+      e = step_E(k, e, wt);
+      r = step_R(k, r, pe[i]);
+      opaque(x[i]);
+      opaque(pe[i]);
+      fence(i);
+    }
+    sr[idx][lc] = r;
+    __syncthreads();
+    const float Rs = enter<NC, LC, false>(Rc, sr, nullptr, rd_full, idx, lc, live);
+    float l = 0.0f, prod = 1.0f;
+    r = Rs;
+#pragma unroll
+    for (int i = 0; i < CK; ++i) {
+      r = step_R(k, r, pe[i]);
+      pe[i] = retention(k, r);  // from here on: eff of the step, and y
+      x[i] = (1.0f - pe[i]) * x[i];
+      l = fmaf(pe[i], l, x[i]);
+      prod *= pe[i];
+      opaque(x[i]);
+      fence(i);
+    }
+    sl[idx][lc] = l;
+    sp[idx][lc] = prod;
+    __syncthreads();
+    l = enter<NC, LC, false>(Lc, sl, sp, 0.0f, idx, lc, live);
+    if (ckpt && ok && mine) keep(seg, l, Es, Rs);
+#pragma unroll
+    for (int i = 0; i < CK; ++i) {
+      l = fmaf(pe[i], l, x[i]);
+      orow.store(i, from_f<E>(l));
+    }
+  }
+  if (tail && wave == 0) {  // the last, shorter chunk: one wave walks it
+    if (ckpt && ok && sub == 0) keep(nfull, Lc, Ec, Rc);
+    const size_t base = static_cast<size_t>(nfull) * CK * H;
+    const Rows<E, BIG> wr(wb + base, H, h, tail, sub * CK), pr(pb + base, H, h, tail, sub * CK),
+        orow(ob + base, H, h, tail, sub * CK);  // past the rows where sub > 0
+    for (int i0 = 0; i0 < tail; i0 += TB) {
+      E wv[TB], pv[TB];
+#pragma unroll
+      for (int i = 0; i < TB; ++i) {  // at clamped rows, all in flight at once
+        wv[i] = wr.load(min(i0 + i, tail - 1));
+        pv[i] = pr.load(min(i0 + i, tail - 1));
+      }
+#pragma unroll
+      for (int i = 0; i < TB; ++i)
+        if (i0 + i < tail) {
+          const float wt = to_f(wv[i]), pe = tanh_abs(fabsf(wt - Ec));
+          Ec = step_E(k, Ec, wt);
+          Rc = step_R(k, Rc, pe);
+          const float eff = retention(k, Rc);
+          Lc = fmaf(eff, Lc, (1.0f - eff) * ((to_f(pv[i]) * pe) * wt));
+          orow.store(i0 + i, from_f<E>(Lc));
+        }
+    }
+  }
+  if (idx == 0 && ok) {
+    LF[ch] = Lc;
+    EF[ch] = Ec;
+    RF[ch] = Rc;
   }
 }
 
-// A sequence of at most one chunk (T <= CK: streaming decode, short query chunks): the
-// three recurrences walked once per channel from the given initial state, in the step
-// order of long.py:492-579 (as phase 3 above), with the final state taken from the walk.
-// The checkpoint (if given) of the one chunk is the initial state.
+// A few steps (streaming decode, T <= kSingle): one thread per channel walks them from the
+// given initial state. The checkpoint (if given) of the one chunk is the initial state.
+constexpr int kSingle = 4;
 template <typename E>
 __global__ void __launch_bounds__(NT) long_fwd_single(int B, int T, int H, int64_t ldx,
                                                       const E* w, const E* p, Logits lg,
@@ -229,8 +384,12 @@ __global__ void __launch_bounds__(NT) long_fwd_single(int B, int T, int H, int64
   }
   for (int t = 0; t < T; ++t) {
     const size_t o = base + static_cast<size_t>(t) * H, io = ibase + static_cast<size_t>(t) * H;
-    float pe, eff;
-    advance(k, ld(w, io), ld(p, io), L, Ev, R, pe, eff);
+    const float wt = ld(w, io), pt = ld(p, io);
+    const float pe = tanh_abs(fabsf(wt - Ev));
+    Ev = step_E(k, Ev, wt);
+    R = step_R(k, R, pe);
+    const float eff = retention(k, R);
+    L = fmaf(eff, L, (1.0f - eff) * ((pt * pe) * wt));
     st(out, o, L);
   }
   LF[ch] = L;
@@ -238,276 +397,224 @@ __global__ void __launch_bounds__(NT) long_fwd_single(int B, int T, int H, int64
   RF[ch] = R;
 }
 
-// Per-channel pass over chunks for state S (0 = L, 1 = E, 2 = R): the chunk-start value
-// goes to the checkpoint slot S; the state after the last chunk to `fin`.
-// x_{k+1} = a_k x_k + loc[k] with a_k = prod[k] (L) or coef^len_k (E: er, R: rd).
-template <int S>
-__global__ void __launch_bounds__(NT) long_fwd_carry(int B, int T, int H, Logits lg,
-                                                     const float* x0, const float* loc,
-                                                     const float* prod, float* ckpt, float* fin) {
-  const int64_t ch = static_cast<int64_t>(blockIdx.x) * NT + threadIdx.x;
-  if (ch >= static_cast<int64_t>(B) * H) return;
-  const Coef k = load_coef(lg.p);
-  const int b = static_cast<int>(ch / H), h = static_cast<int>(ch % H);
-  const int nseg = (T + CK - 1) / CK;
-  const float coef = S == 1 ? k.er : k.rd;
-  const float a_full = powi(coef, CK);
-  float x = x0[ch];
-  for (int kk = 0; kk < nseg; ++kk) {
-    ckpt[(static_cast<size_t>(b) * nseg + kk) * 3 * H + S * H + h] = x;
-    const size_t li = static_cast<size_t>(kk) * B * H + ch;
-    const int len = min(CK, T - kk * CK);
-    const float a = S == 0 ? prod[li] : (len == CK ? a_full : powi(coef, len));
-    x = a * x + loc[li];
-  }
-  fin[ch] = x;
-}
-
-// Backward. Walking time in reverse, one step maps the carried adjoints x = (gL, gR, gE)
-// (coming from step t + 1) to the ones leaving step t, affinely:
-//   gL' = eff (gL + g_t)
-//   gR' = rd gR + rd k a (gL + g_t)                          k = (1 - ret) rs, a = L_{t-1} - sal w
-//   gE' = er gE + s (1 - rd) gR + c (gL + g_t)               s = (1 - pe^2) sign(w - E_{t-1})
-//                                                              c = s ((1 - rd) k a - (1 - eff) w p)
-// i.e. x' = M_t (x + g_t e0) with M_t lower triangular. Over a chunk, x_out = A x_in + v
-// with A = M_0 ... M_{len-1} and v = sum_i (M_0 ... M_{i-1}) M_i g_i e0, both accumulated
-// in forward time order, so one forward pass over each chunk yields its map; a per-channel pass over the chunks then gives the exact
-// adjoints entering each chunk, and a last pass walks each chunk backward with those
-// adjoints to produce gw, gp and the logit partials. Both chunk passes replay the forward
-// recurrence over their chunk from its checkpoint for the values around each step.
-
-// Per-step coefficients of M_t from the forward values around step t.
-struct StepMap {
-  float m00, m10, m11, m20, m21, m22;
-};
-
-__device__ __forceinline__ StepMap step_map(const Coef& k, float wt, float pt, float Lp, float Ep,
-                                            float pe, float eff) {
-  const float kap = (1.0f - k.ret) * k.rs;
-  const float sal = pt * pe;
-  const float a = Lp - sal * wt;
-  const float sgn = (1.0f - pe * pe) * signf_(wt - Ep);
-  StepMap m;
-  m.m00 = eff;
-  m.m10 = k.rd * kap * a;
-  m.m11 = k.rd;
-  m.m20 = sgn * ((1.0f - k.rd) * kap * a - (1.0f - eff) * wt * pt);
-  m.m21 = sgn * (1.0f - k.rd);
-  m.m22 = k.er;
-  return m;
-}
-
-// Chunk maps: A (lower triangular, 6 entries) and v (3 entries), stored component-major
-// in `maps` [9][nseg][B*H]. The forward values around each step are replayed from the
-// chunk's checkpoint.
-template <typename E>
-__global__ void __launch_bounds__(NT) long_bwd_map(int B, int T, int H, int64_t ldx,
-                                                   const E* w, const E* p, Logits lg,
-                                                   const float* ckpt, const E* gout,
-                                                   float* maps) {
-  ChunkIdx c;
-  if (!chunk_idx(B, T, H, ldx, c)) return;
-  const Coef k = load_coef(lg.p);
-  float wv[CK], pv[CK], gv[CK];
-#pragma unroll
-  for (int i = 0; i < CK; ++i) {
-    // Clamped, unconditional loads so all requests are in flight at once (steps past the
-    // chunk end are never used).
-    const size_t t = static_cast<size_t>(c.t0 + min(i, c.len - 1)) * H;
-    wv[i] = ld(w, c.ibase + t);
-    pv[i] = ld(p, c.ibase + t);
-    gv[i] = ld(gout, c.base + t);
-  }
-  float L = ckpt[c.cbase], Ev = ckpt[c.cbase + H], R = ckpt[c.cbase + 2 * H];
-  float p00 = 1.f, p10 = 0.f, p11 = 1.f, p20 = 0.f, p21 = 0.f, p22 = 1.f;
-  float v0 = 0.f, v1 = 0.f, v2 = 0.f;
-#pragma unroll
-  for (int i = 0; i < CK; ++i) {
-    if (i < c.len) {
-      const float Lp = L, Ep = Ev;
-      float pe, eff;
-      advance(k, wv[i], pv[i], L, Ev, R, pe, eff);
-      const StepMap m = step_map(k, wv[i], pv[i], Lp, Ep, pe, eff);
-      // v += P (M_i g_i e0)
-      const float u0 = m.m00 * gv[i], u1 = m.m10 * gv[i], u2 = m.m20 * gv[i];
-      v0 += p00 * u0;
-      v1 += p10 * u0 + p11 * u1;
-      v2 += p20 * u0 + p21 * u1 + p22 * u2;
-      // P = P M_i
-      const float n20 = p20 * m.m00 + p21 * m.m10 + p22 * m.m20;
-      const float n21 = p21 * m.m11 + p22 * m.m21;
-      const float n10 = p10 * m.m00 + p11 * m.m10;
-      p00 *= m.m00;
-      p10 = n10;
-      p11 *= m.m11;
-      p20 = n20;
-      p21 = n21;
-      p22 *= m.m22;
-    }
-  }
-  const size_t stride = static_cast<size_t>(c.nseg) * B * H;
-  const size_t li = static_cast<size_t>(c.k) * B * H + c.ch;
-  maps[li] = p00;
-  maps[li + stride] = p10;
-  maps[li + 2 * stride] = p11;
-  maps[li + 3 * stride] = p20;
-  maps[li + 4 * stride] = p21;
-  maps[li + 5 * stride] = p22;
-  maps[li + 6 * stride] = v0;
-  maps[li + 7 * stride] = v1;
-  maps[li + 8 * stride] = v2;
-}
-
-// Per-channel reverse pass over the chunk maps: x_in(k) = adjoints entering chunk k (from
-// chunk k + 1), written over the map's first three components; x leaving chunk 0 goes to
-// gL0, gR0, gE0.
-__global__ void __launch_bounds__(NT) long_bwd_carry(int B, int T, int H, const float* gLF,
-                                                     const float* gRF, const float* gEF,
-                                                     float* maps, float* gL0, float* gR0,
-                                                     float* gE0) {
-  const int64_t ch = static_cast<int64_t>(blockIdx.x) * NT + threadIdx.x;
-  if (ch >= static_cast<int64_t>(B) * H) return;
-  const int nseg = (T + CK - 1) / CK;
-  const size_t stride = static_cast<size_t>(nseg) * B * H;
-  float x0 = gLF ? gLF[ch] : 0.0f, x1 = gRF ? gRF[ch] : 0.0f, x2 = gEF ? gEF[ch] : 0.0f;
-  for (int kk = nseg - 1; kk >= 0; --kk) {
-    float* m = maps + static_cast<size_t>(kk) * B * H + ch;
-    const float a00 = m[0], a10 = m[stride], a11 = m[2 * stride], a20 = m[3 * stride],
-                a21 = m[4 * stride], a22 = m[5 * stride], v0 = m[6 * stride],
-                v1 = m[7 * stride], v2 = m[8 * stride];
-    m[0] = x0;
-    m[stride] = x1;
-    m[2 * stride] = x2;
-    const float y0 = a00 * x0 + v0;
-    const float y1 = a10 * x0 + a11 * x1 + v1;
-    const float y2 = a20 * x0 + a21 * x1 + a22 * x2 + v2;
-    x0 = y0;
-    x1 = y1;
-    x2 = y2;
-  }
-  gL0[ch] = x0;
-  gR0[ch] = x1;
-  gE0[ch] = x2;
-}
-
-// Final pass: walk the chunk backward from the exact entering adjoints (maps components
-// 0..2), in sub-blocks of SB steps from the last: each sub-block replays its forward steps
-// from its entering states (found by one replay of the chunk from its checkpoint) and keeps
-// them in registers for its backward walk, so a thread holds SB steps of states instead of
-// CK (the replays call `advance`, so every state equals the forward's bit for bit). Writes
-// gw, gp (batch rows ldo apart) and reduces the logit gradients per block (fixed order).
+// Backward. Walking time in reverse with g_t the output's gradient and x_t = sal_t w_t:
+//   gL_t  = g_t + eff_{t+1} gL_{t+1}             (total adjoint of L_t)
+//   deff  = gL_t (L_{t-1} - x_t),  dsal = gL_t (1 - eff_t) w_t
+//   dR_t  = rd dR_{t+1} + deff (1-ret) rs
+//   dpe   = dsal p_t - (1-rd) dR_t,  darg = dpe (1 - pe^2) sign(w_t - E_{t-1})
+//   dE_t  = er dE_{t+1} - darg_{t+1}
+//   gw_t  = gL_t (1 - eff_t) sal_t + darg + (1-er) dE_t,   gp_t = dsal pe
+// three chained recurrences again, with the coefficients eff_t, rd and er. Writes gw, gp (batch
+// rows ldo apart) and one partial of the four logit gradients per workgroup (fixed order).
 // ACC: gw += the gradient rounded to E, the sum formed in fp32 and rounded once (an add of
 // the rounded gradient into an existing gradient buffer).
-constexpr int SB = 8;
-static_assert(CK % SB == 0, "whole sub-blocks per chunk");
+// The wave keeps 7 values per step (w and p of bf16 in one register): at most 256 registers,
+// 8 waves per CU; fp32 workgroups have 4 waves, which may use twice as many.
+template <typename E>
+struct Pair {  // w and p of one step
+  E w, p;
+  __device__ __forceinline__ void set(E a, E b) {
+    w = a;
+    p = b;
+  }
+  __device__ __forceinline__ float fw() const { return to_f(w); }
+  __device__ __forceinline__ float fp() const { return to_f(p); }
+  __device__ __forceinline__ void opaque_() {
+    opaque(w);
+    opaque(p);
+  }
+};
+template <>
+struct Pair<bf16> {
+  uint32_t v;
+  __device__ __forceinline__ void set(bf16 a, bf16 b) { v = static_cast<uint32_t>(a) << 16 | b; }
+  __device__ __forceinline__ float fw() const { return __builtin_bit_cast(float, v & 0xffff0000u); }
+  __device__ __forceinline__ float fp() const { return __builtin_bit_cast(float, v << 16); }
+  __device__ __forceinline__ void opaque_() { opaque(v); }
+};
 
-template <typename E, bool ACC>
-__global__ void __launch_bounds__(NT) long_bwd_final(int B, int T, int H, int64_t ldx,
-                                                     int64_t ldo, const E* w, const E* p,
-                                                     Logits lg, const float* ckpt,
-                                                     const E* gout, const float* maps, E* gw,
-                                                     E* gp, float* part) {
-  constexpr int NSB = CK / SB;
-  __shared__ float red[4][NT];
-  ChunkIdx c;
-  const bool ok = chunk_idx(B, T, H, ldx, c);
+template <typename E, bool ACC, int NW, int G, bool BIG>
+__global__ void __launch_bounds__(NW* LANES, is_bf16<E>::value ? 2 : 1)
+    long_bwd_kernel(int T, int H, int64_t ldx, int64_t ldo, const E* __restrict__ w,
+                    const E* __restrict__ p, Logits lg, const float* __restrict__ ckpt,
+                    const E* __restrict__ gout, const float* __restrict__ gLF,
+                    const float* __restrict__ gRF, const float* __restrict__ gEF,
+                    E* __restrict__ gw, E* __restrict__ gp, float* __restrict__ gL0,
+                    float* __restrict__ gR0, float* __restrict__ gE0, float* __restrict__ part) {
+  constexpr int NC = NW * G, LC = LANES / G;
+  __shared__ float sl[NC][LC], sp[NC][LC], sr[NC][LC], se[NC][LC];
+  __shared__ float red[4][NW];
+  const int lane = threadIdx.x & 63, wave = wave_id();
+  const int lc = lane % LC, sub = lane / LC, idx = wave * G + sub;
+  const int h = blockIdx.x * LC + lc, b = blockIdx.y;
+  const bool ok = h < H;
+  const int hc = ok ? h : H - 1;
   const Coef k = load_coef(lg.p);
-  float d_er = 0.f, d_rd = 0.f, d_ret = 0.f, d_rs = 0.f;
-  if (ok) {
-    const size_t obase = static_cast<size_t>(c.b) * ldo + c.h;
-    float wv[CK], pv[CK];
+  const float er_full = powi(k.er, CK), rd_full = powi(k.rd, CK);
+  const float kap = (1.0f - k.ret) * k.rs;
+  const size_t ch = static_cast<size_t>(b) * H + hc;
+  float gLc = gLF ? gLF[ch] : 0.0f, gRc = gRF ? gRF[ch] : 0.0f, gEc = gEF ? gEF[ch] : 0.0f;
+  E* wb = const_cast<E*>(w) + static_cast<size_t>(b) * ldx;
+  E* pb = const_cast<E*>(p) + static_cast<size_t>(b) * ldx;
+  E* gb = const_cast<E*>(gout) + static_cast<size_t>(b) * T * H;
+  E* gwb = gw + static_cast<size_t>(b) * ldo;
+  E* gpb = gp + static_cast<size_t>(b) * ldo;
+  const int nseg = (T + CK - 1) / CK, nfull = T / CK, tail = T % CK;
+  float t_er = 0.f, t_rd = 0.f, t_ret = 0.f, t_rs = 0.f;
+  auto block = [&](auto full, int k0, int live) {  // as the forward's
+    const int seg = k0 + idx;
+    const bool mine = idx < live;
+    const int wlive = min(max(live - wave * G, 0), G);          // chunks of this wave,
+    const int len = wlive == 0 ? 0 : full ? CK * wlive : tail;  // and their steps
+    const float er_pow = full ? er_full : powi(k.er, tail);
+    const float rd_pow = full ? rd_full : powi(k.rd, tail);
+    const size_t base = static_cast<size_t>(wlive > 0 ? k0 + wave * G : 0) * CK * H;
+    const int first = sub * CK;
+    const Rows<E, BIG> wr(wb + base, H, h, len, first), pr(pb + base, H, h, len, first),
+        grow(gb + base, H, h, len, first), gwr(gwb + base, H, h, len, first),
+        gpr(gpb + base, H, h, len, first);
+    Pair<E> wp[CK];
+    E gr[CK];
 #pragma unroll
     for (int i = 0; i < CK; ++i) {
-      // Clamped, unconditional loads (steps past the chunk end are never used).
-      const size_t t = static_cast<size_t>(c.t0 + min(i, c.len - 1)) * H;
-      wv[i] = ld(w, c.ibase + t);
-      pv[i] = ld(p, c.ibase + t);
+      const int j = full && !BIG ? i : min(i, max(len - 1, 0));
+      wp[i].set(wr.load(j), pr.load(j));
+      gr[i] = grow.load(j);
     }
-    float Ls[NSB], Es[NSB], Rs[NSB];
-    {
-      float L = ckpt[c.cbase], Ev = ckpt[c.cbase + H], R = ckpt[c.cbase + 2 * H];
+    __builtin_amdgcn_sched_barrier(0);
+    const float* c = ckpt + (static_cast<size_t>(b) * nseg + (mine ? seg : 0)) * 3 * H;
+    float L = c[hc], Ev = (c + H)[hc];
+    const float Rs = (c + 2 * static_cast<size_t>(H))[hc];
+    // Replay: per step the difference, pe, a = L - x and R after the step; and, walking back,
+    // the chunk's gL from zero with its product of eff.
+    float diff[CK], pe[CK], a[CK], R[CK], g[CK];
+    float l = 0.0f, prod = 1.0f;
+    auto forget = [&] {
 #pragma unroll
       for (int i = 0; i < CK; ++i) {
-        if (i % SB == 0) {
-          Ls[i / SB] = L;
-          Es[i / SB] = Ev;
-          Rs[i / SB] = R;
-        }
-        if (i < c.len) {
-          float pe, eff;
-          advance(k, wv[i], pv[i], L, Ev, R, pe, eff);
-        }
+        wp[i].opaque_();
+        opaque(R[i]);
+        opaque(gr[i]);
       }
+    };
+    float r = Rs;
+#pragma unroll
+      for (int i = 0; i < CK; ++i)
+        if (full || i < tail) {
+          const float wt = wp[i].fw();
+          diff[i] = wt - Ev;
+          pe[i] = tanh_abs(fabsf(diff[i]));
+          Ev = step_E(k, Ev, wt);
+          r = step_R(k, r, pe[i]);
+          R[i] = r;
+          const float x = (wp[i].fp() * pe[i]) * wt, eff = retention(k, r);
+          a[i] = L - x;
+          L = fmaf(eff, L, (1.0f - eff) * x);
+          opaque(diff[i]);
+          opaque(pe[i]);
+          opaque(a[i]);
+          opaque(R[i]);
+          wp[i].opaque_();
+          fence(i);
+        }
+#pragma unroll
+    for (int i = CK - 1; i >= 0; --i)
+        if (full || i < tail) {
+          const float eff = retention(k, R[i]);
+          l = eff * (l + to_f(gr[i]));
+          prod *= eff;
+          fence(i);
+        }
+    forget();
+    sl[idx][lc] = l;
+    sp[idx][lc] = prod;
+    __syncthreads();
+    l = enter<NC, LC, true>(gLc, sl, sp, 0.0f, idx, lc, live);
+    // gL of every step (in g), deff (in a), the chunk's gR from zero.
+    r = 0.0f;
+#pragma unroll
+    for (int i = CK - 1; i >= 0; --i)
+        if (full || i < tail) {
+          g[i] = l + to_f(gr[i]);
+          l = g[i] * retention(k, R[i]);
+          a[i] = g[i] * a[i];
+          r = fmaf(a[i], kap, r) * k.rd;
+          opaque(g[i]);
+          opaque(a[i]);
+          fence(i);
+        }
+    forget();
+    sr[idx][lc] = r;
+    __syncthreads();
+    r = enter<NC, LC, true>(gRc, sr, nullptr, rd_pow, idx, lc, live);
+    // gp; darg (in pe) and the rest of gw (in g); the chunk's gE from zero.
+    float e = 0.0f, d_er = 0.f, d_rd = 0.f, d_ret = 0.f, d_rs = 0.f;
+#pragma unroll
+    for (int i = CK - 1; i >= 0; --i)
+        if (full || i < tail) {
+          const float wt = wp[i].fw(), pt = wp[i].fp(), pi = pe[i];
+          const float gx = g[i] * (1.0f - retention(k, R[i]));  // gradient of x
+          const float dsal = gx * wt;
+          const float dR = fmaf(a[i], kap, r);
+          r = dR * k.rd;
+          const float dpe = fmaf(dsal, pt, -(dR * (1.0f - k.rd)));
+          const float m = dpe * fmaf(-pi, pi, 1.0f);
+          const float darg = diff[i] == 0.0f ? 0.0f : copysignf(1.0f, diff[i]) * m;
+          d_rd = fmaf(dR, (i > 0 ? R[i - 1] : Rs) - (1.0f - pi), d_rd);
+          d_ret = fmaf(a[i], fmaf(-k.rs, R[i], 1.0f), d_ret);
+          d_rs = fmaf(a[i], R[i], d_rs);
+          e = fmaf(k.er, e, -darg);
+          g[i] = fmaf(gx, pt * pi, darg);
+          pe[i] = darg;
+          opaque(g[i]);
+          opaque(pe[i]);
+          gpr.store(i, from_f<E>(dsal * pi));
+          if (i % 4 == 0) __builtin_amdgcn_sched_barrier(0);
+        }
+    E sv[ACC ? CK : 1];
+    if constexpr (ACC) {
+#pragma unroll
+      for (int i = 0; i < CK; ++i) sv[i] = gwr.load(full && !BIG ? i : min(i, max(len - 1, 0)));
     }
-    const size_t stride = static_cast<size_t>(c.nseg) * B * H;
-    const size_t li = static_cast<size_t>(c.k) * B * H + c.ch;
-    float gLc = maps[li], gRc = maps[li + stride], gEc = maps[li + 2 * stride];
+    se[idx][lc] = e;
+    __syncthreads();
+    e = enter<NC, LC, true>(gEc, se, nullptr, er_pow, idx, lc, live);
 #pragma unroll
-    for (int sb = NSB - 1; sb >= 0; --sb) {
-      float gv[SB], sv[ACC ? SB : 1], Lv[SB], Ev[SB], Rv[SB];
-#pragma unroll
-      for (int j = 0; j < SB; ++j) {
-        const size_t t = static_cast<size_t>(c.t0 + min(sb * SB + j, c.len - 1)) * H;
-        gv[j] = ld(gout, c.base + t);
-        if constexpr (ACC) sv[j] = ld(gw, obase + t);
-      }
-      float L = Ls[sb], Es_ = Es[sb], R = Rs[sb];
-#pragma unroll
-      for (int j = 0; j < SB; ++j) {
-        const int i = sb * SB + j;
-        Lv[j] = L;
-        Ev[j] = Es_;
-        Rv[j] = R;
-        if (i < c.len) {
-          float pe, eff;
-          advance(k, wv[i], pv[i], L, Es_, R, pe, eff);
+    for (int i = CK - 1; i >= 0; --i)
+        if (full || i < tail) {
+          float v = fmaf(1.0f - k.er, e, g[i]);
+          if constexpr (ACC) v = to_f(sv[i]) + round_to<E>(v);
+          d_er = fmaf(-e, diff[i], d_er);
+          e = fmaf(k.er, e, -pe[i]);
+          gwr.store(i, from_f<E>(v));
         }
-      }
-#pragma unroll
-      for (int j = SB - 1; j >= 0; --j) {
-        const int i = sb * SB + j;
-        if (i < c.len) {
-          const float wt = wv[i], pt = pv[i];
-          const float diff = wt - Ev[j];
-          const float pe = tanhf(fabsf(diff));
-          const float sal = pt * pe;
-          const float Rcur = k.rd * Rv[j] + (1.0f - k.rd) * (1.0f - pe);
-          const float eff = k.ret + (1.0f - k.ret) * k.rs * Rcur;
-          const float gL = gv[j] + gLc;
-          const float deff = gL * (Lv[j] - sal * wt);
-          const float dsal = gL * (1.0f - eff) * wt;
-          gLc = gL * eff;
-          const float dR = gRc + deff * (1.0f - k.ret) * k.rs;
-          gRc = dR * k.rd;
-          const float dpe = dsal * pt - dR * (1.0f - k.rd);
-          const float darg = dpe * (1.0f - pe * pe) * signf_(diff);
-          const float dE = gEc;
-          gEc = k.er * dE - darg;
-          const size_t o = obase + static_cast<size_t>(c.t0 + i) * H;
-          st(gp, o, dsal * pe);
-          const float gwv = gL * (1.0f - eff) * sal + darg + (1.0f - k.er) * dE;
-          if constexpr (ACC)
-            st(gw, o, sv[j] + round_to<E>(gwv));
-          else
-            st(gw, o, gwv);
-          d_er += dE * (Ev[j] - wt);
-          d_rd += dR * (Rv[j] - (1.0f - pe));
-          d_ret += deff * (1.0f - k.rs * Rcur);
-          d_rs += deff * (1.0f - k.ret) * Rcur;
-        }
-      }
-    }
+    t_er += mine ? d_er : 0.0f;
+    t_rd += mine ? d_rd : 0.0f;
+    t_ret += mine ? d_ret : 0.0f;
+    t_rs += mine ? d_rs : 0.0f;
+  };
+  if (tail) block(std::false_type{}, nfull, 1);
+  for (int k0 = nfull > 0 ? (nfull - 1) / NC * NC : -1; k0 >= 0; k0 -= NC)
+    block(std::true_type{}, k0, min(NC, nfull - k0));
+  if (idx == 0 && ok) {
+    gL0[ch] = gLc;
+    gR0[ch] = gRc;
+    gE0[ch] = gEc;
   }
-  // d logit = d coef * sigmoid'(logit), reduced per block in a fixed order.
-  red[0][threadIdx.x] = d_er * k.er * (1.0f - k.er);
-  red[1][threadIdx.x] = d_rd * k.rd * (1.0f - k.rd);
-  red[2][threadIdx.x] = d_ret * k.ret * (1.0f - k.ret);
-  red[3][threadIdx.x] = d_rs * k.rs * (1.0f - k.rs);
+  // d logit = d coef * sigmoid'(logit), reduced per workgroup in a fixed order.
+  const float d[4] = {t_er * k.er * (1.0f - k.er), t_rd * k.rd * (1.0f - k.rd),
+                      t_ret * k.ret * (1.0f - k.ret),
+                      t_rs * (1.0f - k.ret) * k.rs * (1.0f - k.rs)};
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const float sum = wave_sum(ok ? d[i] : 0.0f);
+    if (lane == 0) red[i][wave] = sum;
+  }
   __syncthreads();
   if (threadIdx.x < 4) {
-    float s = 0.0f;
-    for (int i = 0; i < NT; ++i) s += red[threadIdx.x][i];
-    part[(static_cast<size_t>(blockIdx.y) * gridDim.x + blockIdx.x) * 4 + threadIdx.x] = s;
+    float sum = 0.0f;
+    for (int i = 0; i < NW; ++i) sum += red[threadIdx.x][i];
+    part[(static_cast<size_t>(b) * gridDim.x + blockIdx.x) * 4 + threadIdx.x] = sum;
   }
 }
 
@@ -524,52 +631,87 @@ using namespace dabsn::longmem;
                     (B) * (H) < (1ll << 31) && (T) < (1ll << 30),                            \
                 "bad shape B=%lld T=%lld H=%lld", (long long)(B), (long long)(T), (long long)(H))
 
+constexpr int kBigRow = 1 << 24;  // see Rows
+
+// Chunks per wave. A workgroup of 64 channels walks T serially, so few channels leave most CUs
+// idle: up to kFew such workgroups a wave takes 4 chunks of 16 channels instead, 4 times the
+// workgroups and a quarter of the blocks (at accesses of 32 bytes, which so few channels can
+// afford). Backward, bf16: B=1, T=4096, H=64 takes 184 us with 64 channels and 85 with 16 (the
+// earlier kernels, parallel over all chunks of T: 78); B=8, T=2573, H=400 (56 workgroups) 134
+// and 99 (117); B=32, T=3200, H=256 (128 workgroups) 175 and 187 (217).
+constexpr int64_t kFew = 64;
+static int wave_chunks(int64_t B, int64_t T, int64_t H) {
+  return B * ((H + LANES - 1) / LANES) <= kFew && T >= 4 * CK ? 4 : 1;
+}
+static int channel_tiles(int64_t B, int64_t T, int64_t H) {
+  const int lc = LANES / wave_chunks(B, T, H);
+  return static_cast<int>((H + lc - 1) / lc);
+}
+
+// Waves per workgroup: as many as there are chunks, up to 8 in the forward (two workgroups per
+// CU, one's arithmetic over the other's loads) and 4 in the backward (the same at its 256
+// registers; one workgroup of 8 waves took 512 us for the shape below). In the bf16 backward 8
+// where every CU has at most one workgroup anyway: B=32, T=3200, H=256 229 -> 175 us.
+// B=16, T=4096, H=2048 bf16: 637 -> 230 us (805 MB: 3.5 TB/s).
 template <typename E>
 static int long_fwd_impl(int B, int T, int H, int64_t ldx, const E* w, const E* p, Logits lg,
-                         const float* L0,
-                         const float* E0, const float* R0, E* out, float* LF, float* EF, float* RF,
-                         float* keep, float* ws, hipStream_t stream) {
-  const int gx = grid_for(B, H);
-  const int nseg = (T + CK - 1) / CK;
-  float* loc0 = ws;
-  float* loc1 = ws + static_cast<size_t>(nseg) * B * H;
-  // [B][nseg][3][H]: the caller's buffer when it keeps the checkpoint, else the workspace.
-  float* ckpt = keep ? keep : ws + 2 * static_cast<size_t>(nseg) * B * H;
-  const dim3 cg(gx, nseg), blk(NT);
-  if (nseg == 1) {  // one chunk: a single walk, no chunk-parallel passes
-    hipLaunchKernelGGL((long_fwd_single<E>), dim3(gx), blk, 0, stream, B, T, H, ldx, w, p, lg, L0, E0,
-                       R0, out, LF, EF, RF, keep);
+                         const float* L0, const float* E0, const float* R0, E* out, float* LF,
+                         float* EF, float* RF, float* keep, hipStream_t stream) {
+  if (T > 0 && T <= kSingle) {
+    hipLaunchKernelGGL((long_fwd_single<E>), dim3(grid_for(B, H)), dim3(NT), 0, stream, B, T, H, ldx,
+                       w, p, lg, L0, E0, R0, out, LF, EF, RF, keep);
     DABSN_HIP_CHECK(hipGetLastError());
     return DABSN_OK;
   }
-  if (nseg > 0) hipLaunchKernelGGL((long_fwd_chunk<E, 0>), cg, blk, 0, stream, B, T, H, ldx, w, p, lg, ckpt, loc0, loc1, out);
-  hipLaunchKernelGGL(long_fwd_carry<1>, dim3(gx), blk, 0, stream, B, T, H, lg, E0, loc0, loc1, ckpt, EF);
-  if (nseg > 0) hipLaunchKernelGGL((long_fwd_chunk<E, 1>), cg, blk, 0, stream, B, T, H, ldx, w, p, lg, ckpt, loc0, loc1, out);
-  hipLaunchKernelGGL(long_fwd_carry<2>, dim3(gx), blk, 0, stream, B, T, H, lg, R0, loc0, loc1, ckpt, RF);
-  if (nseg > 0) hipLaunchKernelGGL((long_fwd_chunk<E, 2>), cg, blk, 0, stream, B, T, H, ldx, w, p, lg, ckpt, loc0, loc1, out);
-  hipLaunchKernelGGL(long_fwd_carry<0>, dim3(gx), blk, 0, stream, B, T, H, lg, L0, loc0, loc1, ckpt, LF);
-  if (nseg > 0) hipLaunchKernelGGL((long_fwd_chunk<E, 3>), cg, blk, 0, stream, B, T, H, ldx, w, p, lg, ckpt, loc0, loc1, out);
+  const int nseg = (T + CK - 1) / CK;
+  const dim3 grid(channel_tiles(B, T, H), B);
+  const bool split = wave_chunks(B, T, H) == 4;
+#define DABSN_LONG(NW, G, BIG)                                                               \
+  hipLaunchKernelGGL((long_fwd_kernel<E, NW, G, BIG>), grid, dim3(NW * LANES), 0, stream, T, H, ldx, \
+                     w, p, lg, L0, E0, R0, out, LF, EF, RF, keep)
+  if (H >= kBigRow)
+    DABSN_LONG(4, 1, true);
+  else if (split && nseg <= 16)
+    DABSN_LONG(4, 4, false);
+  else if (split)
+    DABSN_LONG(8, 4, false);
+  else if (nseg <= 1)
+    DABSN_LONG(1, 1, false);
+  else if (nseg <= 2)
+    DABSN_LONG(2, 1, false);
+  else if (nseg <= 4)
+    DABSN_LONG(4, 1, false);
+  else
+    DABSN_LONG(8, 1, false);
+#undef DABSN_LONG
   DABSN_HIP_CHECK(hipGetLastError());
   return DABSN_OK;
 }
 
-template <typename E>
+// B=16, T=4096, H=2048 bf16: 891 -> 482 us (1.39 GB: 2.9 TB/s).
+template <typename E, bool ACC>
 static int long_bwd_impl(int B, int T, int H, int64_t ldx, const E* w, const E* p, Logits lg,
                          const float* ckpt, const E* gout, const float* gLF, const float* gEF,
-                         const float* gRF, E* gw, E* gp, int64_t ldo, bool acc, float* gL0,
-                         float* gE0, float* gR0, float* part, float* ws, hipStream_t stream) {
-  const int gx = grid_for(B, H);
+                         const float* gRF, E* gw, E* gp, int64_t ldo, float* gL0, float* gE0,
+                         float* gR0, float* part, hipStream_t stream) {
   const int nseg = (T + CK - 1) / CK;
-  const dim3 cg(gx, nseg), blk(NT);
-  if (nseg > 0)
-    hipLaunchKernelGGL(long_bwd_map<E>, cg, blk, 0, stream, B, T, H, ldx, w, p, lg, ckpt, gout,
-                       ws);
-  hipLaunchKernelGGL(long_bwd_carry, dim3(gx), blk, 0, stream, B, T, H, gLF, gRF, gEF, ws, gL0,
-                     gR0, gE0);
-  auto final_pass = acc ? long_bwd_final<E, true> : long_bwd_final<E, false>;
-  if (nseg > 0)
-    hipLaunchKernelGGL(final_pass, cg, blk, 0, stream, B, T, H, ldx, ldo, w, p, lg, ckpt, gout,
-                       ws, gw, gp, part);
+  const dim3 grid(channel_tiles(B, T, H), B);
+#define DABSN_LONG(NW, G, BIG)                                                                  \
+  hipLaunchKernelGGL((long_bwd_kernel<E, ACC, NW, G, BIG>), grid, dim3(NW * LANES), 0, stream, T, H, \
+                     ldx, ldo, w, p, lg, ckpt, gout, gLF, gRF, gEF, gw, gp, gL0, gR0, gE0, part)
+  if (H >= kBigRow)
+    DABSN_LONG(4, 1, true);
+  else if (wave_chunks(B, T, H) == 4)
+    DABSN_LONG(4, 4, false);
+  else if (nseg <= 1)
+    DABSN_LONG(1, 1, false);
+  else if (nseg <= 2)
+    DABSN_LONG(2, 1, false);
+  else if (nseg <= 4 || static_cast<int64_t>(grid.x) * B > 256 || !is_bf16<E>::value)
+    DABSN_LONG(4, 1, false);
+  else if constexpr (is_bf16<E>::value)
+    DABSN_LONG(8, 1, false);
+#undef DABSN_LONG
   DABSN_HIP_CHECK(hipGetLastError());
   return DABSN_OK;
 }
@@ -621,12 +763,8 @@ int dabsn_hip_linrec_bwd(int dtype, int64_t B, int64_t T, int64_t H, const void*
   return DABSN_OK;
 }
 
-size_t dabsn_hip_long_workspace_bytes(int64_t B, int64_t T, int64_t H, int backward) {
-  const int64_t nseg = (T + CK - 1) / CK;
-  // forward: two chunk-end arrays + the chunk-start checkpoint (3 per chunk; used when the
-  // caller passes no checkpoint buffer of its own);
-  // backward: the 9-component chunk maps.
-  return static_cast<size_t>(backward ? 9 : 5) * static_cast<size_t>(nseg) * B * H * sizeof(float);
+size_t dabsn_hip_long_workspace_bytes(int64_t, int64_t, int64_t, int) {
+  return 0;  // the chunk ends stay in LDS
 }
 
 // Batch stride of [B, T, H] operands: ldx elements (0: T H, the contiguous layout); at least
@@ -646,30 +784,24 @@ int dabsn_hip_long_fwd(int dtype, int64_t B, int64_t T, int64_t H, int64_t ldx, 
   const int64_t lx = batch_stride(B, T, H, ldx);
   DABSN_REQUIRE(lx >= 0, "long scan: bad input batch stride %lld for T=%lld H=%lld",
                 (long long)ldx, (long long)T, (long long)H);
-  DABSN_REQUIRE(w && p && logits && L0 && E0 && R0 && (out || T == 0) && LF && EF && RF &&
-                    (workspace || T == 0),
+  DABSN_REQUIRE(w && p && logits && L0 && E0 && R0 && (out || T == 0) && LF && EF && RF,
                 "long scan: null pointer");
+  (void)workspace;
+  (void)workspace_bytes;
   for (int i = 0; i < 4; ++i) DABSN_REQUIRE(logits[i], "long scan: null logit %d", i);
-  DABSN_REQUIRE(workspace_bytes >= dabsn_hip_long_workspace_bytes(B, T, H, 0),
-                "long scan: workspace %zu B < required %zu B", workspace_bytes,
-                dabsn_hip_long_workspace_bytes(B, T, H, 0));
   DABSN_REQUIRE((T + CK - 1) / CK < 65536, "long scan: T too long");
   Logits lg{{logits[0], logits[1], logits[2], logits[3]}};
   if (dtype == kBF16)
     return long_fwd_impl<bf16>((int)B, (int)T, (int)H, lx, (const bf16*)w, (const bf16*)p, lg,
-                               L0, E0, R0, (bf16*)out, LF, EF, RF, ckpt, (float*)workspace,
-                               stream);
+                               L0, E0, R0, (bf16*)out, LF, EF, RF, ckpt, stream);
   if (dtype == kF32)
     return long_fwd_impl<float>((int)B, (int)T, (int)H, lx, (const float*)w, (const float*)p, lg,
-                                L0, E0, R0, (float*)out, LF, EF, RF, ckpt, (float*)workspace,
-                                stream);
+                                L0, E0, R0, (float*)out, LF, EF, RF, ckpt, stream);
   DABSN_REQUIRE(false, "long scan: bad dtype %d", dtype);
   return DABSN_OK;
 }
 
-int64_t dabsn_hip_long_partials(int64_t B, int64_t T, int64_t H) {
-  return static_cast<int64_t>(grid_for(B, H)) * ((T + CK - 1) / CK);
-}
+int64_t dabsn_hip_long_partials(int64_t B, int64_t T, int64_t H) { return B * channel_tiles(B, T, H); }
 
 int dabsn_hip_long_bwd(int dtype, int64_t B, int64_t T, int64_t H, int64_t ldx, const void* w,
                        const void* p, const float* const* logits, const float* ckpt,
@@ -683,24 +815,26 @@ int dabsn_hip_long_bwd(int dtype, int64_t B, int64_t T, int64_t H, int64_t ldx, 
                 "long scan backward: bad batch stride (inputs %lld, outputs %lld) for T=%lld "
                 "H=%lld", (long long)ldx, (long long)ldo, (long long)T, (long long)H);
   DABSN_REQUIRE(w && p && logits && (ckpt || T == 0) && (gout || T == 0) && gL0 && gE0 && gR0 &&
-                    (part_logit || T == 0) && (workspace || T == 0) && ((gw && gp) || T == 0),
+                    part_logit && ((gw && gp) || T == 0),
                 "long scan backward: null pointer");
+  (void)workspace;
+  (void)workspace_bytes;
   for (int i = 0; i < 4; ++i) DABSN_REQUIRE(logits[i], "long scan backward: null logit %d", i);
-  DABSN_REQUIRE(workspace_bytes >= dabsn_hip_long_workspace_bytes(B, T, H, 1),
-                "long scan backward: workspace %zu B < required %zu B", workspace_bytes,
-                dabsn_hip_long_workspace_bytes(B, T, H, 1));
   DABSN_REQUIRE((T + CK - 1) / CK < 65536, "long scan backward: T too long");
   Logits lg{{logits[0], logits[1], logits[2], logits[3]}};
-  if (dtype == kBF16)
-    return long_bwd_impl<bf16>((int)B, (int)T, (int)H, lx, (const bf16*)w, (const bf16*)p, lg,
-                               ckpt, (const bf16*)gout, gLF, gEF, gRF, (bf16*)gw, (bf16*)gp, lo,
-                               gw_accumulate != 0, gL0, gE0, gR0, part_logit, (float*)workspace,
-                               stream);
-  if (dtype == kF32)
-    return long_bwd_impl<float>((int)B, (int)T, (int)H, lx, (const float*)w, (const float*)p, lg,
-                                ckpt, (const float*)gout, gLF, gEF, gRF, (float*)gw, (float*)gp,
-                                lo, gw_accumulate != 0, gL0, gE0, gR0, part_logit,
-                                (float*)workspace, stream);
+#define DABSN_LONG_BWD(E, ACC)                                                                 \
+  return long_bwd_impl<E, ACC>((int)B, (int)T, (int)H, lx, (const E*)w, (const E*)p, lg, ckpt,   \
+                               (const E*)gout, gLF, gEF, gRF, (E*)gw, (E*)gp, lo, gL0, gE0, gR0, \
+                               part_logit, stream)
+  if (dtype == kBF16) {
+    if (gw_accumulate) DABSN_LONG_BWD(bf16, true);
+    DABSN_LONG_BWD(bf16, false);
+  }
+  if (dtype == kF32) {
+    if (gw_accumulate) DABSN_LONG_BWD(float, true);
+    DABSN_LONG_BWD(float, false);
+  }
+#undef DABSN_LONG_BWD
   DABSN_REQUIRE(false, "long scan backward: bad dtype %d", dtype);
   return DABSN_OK;
 }

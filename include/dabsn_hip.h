@@ -175,7 +175,7 @@ int dabsn_hip_linrec_bwd(int dtype, int64_t B, int64_t T, int64_t H, const void*
  * read.py:625-636). logits[4] point at fp32 scalars (logit_expect_retain,
  * logit_retention_decay, logit_retain, logit_retention_strength). State L0/E0/R0 [B,H]
  * fp32 in, LF/EF/RF out. Both directions are chunked over time (chunks of DABSN_LONG_CKPT
- * steps) and need dabsn_hip_long_workspace_bytes() bytes of workspace. `ckpt` (may be NULL)
+ * steps) and need dabsn_hip_long_workspace_bytes() bytes of workspace (0: none). `ckpt` (may be NULL)
  * receives the checkpoint the backward replays each chunk from: the fp32 states entering
  * every chunk, [B][ceil(T / DABSN_LONG_CKPT)][3][H] = (L, E, R). `ldx`: elements between
  * the batch rows of w and p (0: T H, contiguous; otherwise >= T H, e.g. a time window of

@@ -302,6 +302,57 @@ def test_long_scan_and_linear_recurrence_match_oracle(cuda_device, T):
         assert_rel(x, y, 1e-6, n)
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("B,T,H", [(2, 4, 1), (2, 5, 63), (3, 31, 65), (2, 63, 64), (1, 65, 130),
+                                   (2, 127, 33), (2, 128, 15), (3, 129, 17), (1, 511, 64),
+                                   (2, 513, 16), (2, 1057, 70), (33, 128, 65), (65, 289, 3),
+                                   (257, 161, 2)])
+def test_long_scan_block_edges(cuda_device, dtype, B, T, H):
+    """Chunk, block and channel-tile edges of the 64- and the 16-channel split, in time windows
+    of longer tapes, against the oracle on the same inputs. The bf16 outputs are rounded once
+    more: at most half an ulp of 8 significant bits, 2^-8 of the value. An accumulated gradient is the plain one added, and a
+    NaN leaves earlier steps and other channels as they are, bit for bit."""
+    g = torch.Generator().manual_seed(T + H)
+    wide = (torch.randn(B, T + 3, H, generator=g) * 0.7).to(dtype).to(cuda_device)
+    w, p = wide[:, 2:T + 2], torch.rand(B, T + 3, H, generator=g).to(dtype).to(cuda_device)[:, 2:T + 2]
+    logits = [torch.tensor([v]) for v in (2.2, 2.0, 2.4, 1.4)]
+    coef = torch.sigmoid(torch.stack([x[0] for x in logits]))
+    L0, E0, R0 = (0.1 * torch.randn(B, H, generator=g) + o for o in (0.0, 0.0, 1.0))
+    d = lambda t: t.to(cuda_device)  # noqa: E731
+    lg = [d(x) for x in logits]
+    tol = 1e-5 if dtype == torch.float32 else 2.0 ** -8 + 1e-5
+    out = ops.long_scan_window(w, p, lg, d(L0), d(E0), d(R0))
+    ref, fin = oracle.long_fwd(np32(w), np32(p), np32(coef), np32(L0), np32(E0), np32(R0))
+    assert_rel(out[0], ref, tol, "long")
+    for n, a, b in zip("LER", out[1:4], fin):
+        assert_rel(a, b, 1e-5, f"final {n}")
+    gout = d(torch.randn(B, T, H, generator=g).to(dtype))
+    gf = [torch.randn(B, H, generator=g) for _ in range(3)]
+    gw, gp, g0, gcoef = oracle.long_bwd(np32(w), np32(p), np32(coef), np32(L0), np32(E0),
+                                        np32(R0), np32(gout), [np32(x) for x in gf])
+    up = (out[4], gout, *[d(x) for x in gf])
+    res = ops.long_scan_backward_parts(w, p, lg, *up)
+    assert_rel(res[0], gw, tol, "g_write")
+    assert_rel(res[1], gp, tol, "g_plasticity")
+    glog = gcoef * np32(coef) * (1 - np32(coef))
+    for i in range(4):
+        assert abs(float(res[2][i]) - glog[i]) <= 1e-4 * max(abs(glog[i]), 1.0)
+    for n, a, b in zip("LER", res[3], (g0[0], g0[1], g0[2])):
+        assert_rel(a, b, 1e-5, f"g {n}0")
+    gw_into, gp_into = torch.randn_like(wide), torch.empty_like(wide)
+    want = gw_into.clone()
+    want[:, 2:T + 2] += res[0]
+    ops.long_scan_backward_parts(w, p, lg, *up, gw_into[:, 2:T + 2], gp_into[:, 2:T + 2])
+    assert torch.equal(gw_into, want) and torch.equal(gp_into[:, 2:T + 2], res[1])
+    t, h = T * 2 // 3, H // 2
+    bad = w.clone()
+    bad[:, t, h] = float("nan")
+    got = ops.long_scan_window(bad, p.contiguous(), lg, d(L0), d(E0), d(R0))[0]
+    keep = torch.arange(H, device=got.device) != h
+    assert torch.equal(got[:, :t], out[0][:, :t]) and bool(got[:, t:, h].isnan().all())
+    assert torch.equal(got[:, :, keep], out[0][:, :, keep])
+
+
 @pytest.mark.parametrize("whole", [0, 1])
 @pytest.mark.parametrize("T", [1, 255, 256, 257, 3000, 16384])
 def test_bank_select_bit_exact(cuda_device, T, whole):
