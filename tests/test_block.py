@@ -121,6 +121,31 @@ def test_forward_query_bank_matches_oracle_unified_read_gpu(cuda_device):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("T", [1, 8, 9, 33, 257])
+@pytest.mark.parametrize("geometry,window", [("seq", -2.0), ("seq", 8.0), ("field", -2.0),
+                                             ("field", 8.0), ("hybrid", 8.0)])
+def test_read_without_autograd_matches_cpu_oracle(cuda_device, geometry, window, T):
+    """Without autograd, the read over banks whose successor rows are bank rows (every position
+    admitted) and are not (a narrow window), at the edge of the streaming read (8 rows) and of
+    a 256-row tile, against the same module on the CPU oracle kernels."""
+    torch.manual_seed(5)
+    B, H = 2, 40
+    read = dabsn_amd.DABSNRead(H, read_geometry=geometry)
+    with torch.no_grad():
+        read.admit_window.fill_(window)
+    g = torch.Generator().manual_seed(T)
+    tapes = [torch.randn(B, T, H, generator=g) for _ in range(3)]
+    tapes += [torch.rand(B, T, H, generator=g) for _ in range(5)]
+    tapes[3] = tapes[5] * tapes[2]
+    dev = copy.deepcopy(read).to(cuda_device)
+    with torch.no_grad():
+        want = read(*tapes)
+        got = dev(*[t.to(cuda_device) for t in tapes])
+    assert dev.last_n_max == read.last_n_max and (window < 0 or read.last_n_max == T)
+    assert rel_err(got.cpu(), want) <= 1e-5
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("geometry", ["field", "hybrid"])
 def test_field_and_hybrid_read_gpu_match_cpu_oracle(cuda_device, geometry):
     """The field and hybrid reads at T=300 (several 256-row tiles, a partially admitted
