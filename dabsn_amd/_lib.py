@@ -13,7 +13,7 @@ import threading
 from pathlib import Path
 
 LIB_PATH = Path(__file__).resolve().parent / "_build" / "libdabsn_hip.so"
-ABI_VERSION = 19
+ABI_VERSION = 20
 
 _lock = threading.Lock()
 _lib = None
@@ -32,6 +32,7 @@ class CoreParams(ctypes.Structure):
 
 
 PTR4 = vp * 4
+PTR19 = vp * 19
 PTR8 = vp * 8
 
 
@@ -83,6 +84,7 @@ _SIGNATURES = {
         [i32, i64, i64, i64, i64, vp, i64, i32, vp, vp, vp, vp, vp], i32),
     "dabsn_hip_core_scan_fwd_call": ([ctypes.POINTER(CoreFwdCall), vp], i32),
     "dabsn_hip_core_scan_bwd_call": ([ctypes.POINTER(CoreBwdCall), vp], i32),
+    "dabsn_hip_core_scan_param_grads": ([i64, i64, i64, vp, vp, PTR19, vp], i32),
     "dabsn_hip_linrec_fwd": ([i32, i64, i64, i64, vp, vp, vp, vp, vp], i32),
     "dabsn_hip_linrec_workspace_bytes": ([i32, i64, i64, i64], sz),
     "dabsn_hip_linrec_bwd": ([i32, i64, i64, i64, vp, vp, vp, vp, vp, vp, vp, vp, sz, vp], i32),

@@ -517,17 +517,18 @@ def core_scan_batched_backward(
     _lib.check(rc, "core scan backward")
     _record_error_word(ws, "core scan backward")
     del keep
-    gvec = part_vec.sum(0)
-    gscal = part_scal.sum(0)
+    gpar = [torch.empty((H,) if i < 16 else (), device=U.device, dtype=torch.float32)
+            for i in range(19)]
+    _lib.check(lib.dabsn_hip_core_scan_param_grads(
+        nbg.value, nwg.value, H, _p(part_vec), _p(part_scal),
+        _lib.PTR19(*[x.data_ptr() for x in gpar]), _stream(U)), "core scan parameter gradients")
     # grad [Ug; A] = [gWgx; day]^T y: one plain GEMM per half (hipBLASLt through torch).
     tk = KernelTimer.begin("core_weight_grad_gemm", U)
     y = U[..., :H].to(dt).reshape(B * T, H)
     gUg = (gWgx.reshape(B * T, H).t() @ y).float()
     gA = (day.reshape(B * T, H).t() @ y).float()
     KernelTimer.end(tk)
-    # operator outputs must not alias each other: split into separate tensors
-    return [gWx, gWgx, gUg, gA, *[gvec[i].clone() for i in range(16)],
-            *[gscal[i].clone() for i in range(3)], gb0, ge0, gc0]
+    return [gWx, gWgx, gUg, gA, *gpar, gb0, ge0, gc0]
 
 
 @core_scan_batched_backward.register_fake

@@ -17,7 +17,7 @@
 #include <stddef.h>
 #include <stdint.h>
 
-#define DABSN_HIP_ABI_VERSION 19
+#define DABSN_HIP_ABI_VERSION 20
 
 /* Status codes returned by every entry point. */
 #define DABSN_OK 0
@@ -145,6 +145,11 @@ typedef struct dabsn_core_bwd_call {
 
 int dabsn_hip_core_scan_fwd_call(const dabsn_core_fwd_call* fwd, hipStream_t stream);
 int dabsn_hip_core_scan_bwd_call(const dabsn_core_bwd_call* bwd, hipStream_t stream);
+/* Sums a reverse scan's partials, part_vec [nbg][16][H] and part_scal [nwg][3], in a fixed
+ * order: out[0..15] receive [H] each, out[16..18] one value each (fp32). */
+int dabsn_hip_core_scan_param_grads(int64_t nbg, int64_t nwg, int64_t H, const float* part_vec,
+                                    const float* part_scal, float* const* out,
+                                    hipStream_t stream);
 
 /* Two streams on complementary halves of the device's CUs (hipExtStreamCreateWithCUMask;
  * on MI355X each gets 16 CUs of every XCD), for overlapping the persistent core scan

@@ -302,6 +302,23 @@ def test_long_scan_and_linear_recurrence_match_oracle(cuda_device, T):
         assert_rel(x, y, 1e-6, n)
 
 
+@pytest.mark.parametrize("nbg,nwg,H", [(1, 1, 1), (3, 4, 255), (4, 256, 256), (7, 257, 257),
+                                       (9, 1029, 40)])
+def test_core_scan_param_grad_sums(cuda_device, nbg, nwg, H):
+    """The partial sums against 64 bits: n additions round by at most n 2^-24 sum |x|."""
+    g = torch.Generator().manual_seed(nbg)
+    vec, scal = torch.randn(nbg, 16, H, generator=g), torch.randn(nwg, 3, generator=g)
+    dv, ds = vec.to(cuda_device), scal.to(cuda_device)
+    outs = [torch.full((H,) if i < 16 else (), float("nan"), device=cuda_device) for i in range(19)]
+    lib = ops._lib.load()
+    ops._lib.check(lib.dabsn_hip_core_scan_param_grads(
+        nbg, nwg, H, dv.data_ptr(), ds.data_ptr(), ops._lib.PTR19(*[o.data_ptr() for o in outs]),
+        ops._stream(dv)), "sums")
+    for got, x in zip(outs, [*vec.double().unbind(1), *scal.double().unbind(1)]):
+        bound = x.shape[0] * 2.0 ** -24 * x.abs().sum(0)
+        assert bool(((got.cpu().double() - x.sum(0)).abs() <= bound).all())
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("B,T,H", [(2, 4, 1), (2, 5, 63), (3, 31, 65), (2, 63, 64), (1, 65, 130),
                                    (2, 127, 33), (2, 128, 15), (3, 129, 17), (1, 511, 64),
