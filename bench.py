@@ -454,7 +454,8 @@ def primitives_main(args):
         "local_field_scatter": ("hbm", 4.0 * FB * cells * D * (9 + 1)),
         # per launch: one 2**24-element chunk (524 rows of 32000)
         "ce_rows_fwd": ("hbm", 2.0 * (1 << 24) // V * V),
-        "ce_rows_bwd": ("hbm", 6.0 * (1 << 24) // V * V),
+        # the bf16 backward reads the logits and writes three bf16 planes
+        "ce_rows_bwd": ("hbm", 8.0 * (1 << 24) // V * V),
     }
     out = {}
     for name, (bound, amount) in work.items():
