@@ -319,6 +319,34 @@ def test_core_scan_param_grad_sums(cuda_device, nbg, nwg, H):
         assert bool(((got.cpu().double() - x.sum(0)).abs() <= bound).all())
 
 
+@pytest.mark.parametrize("dtype,B,T,H", [(torch.bfloat16, 4, 16, 4096), (torch.bfloat16, 4, 2, 4096),
+                                         (torch.bfloat16, 17, 9, 2048), (torch.float32, 9, 5, 300)])
+def test_core_scan_reads_and_returns_only_what_it_wrote(cuda_device, dtype, B, T, H):
+    """Freed memory full of NaN under every buffer a scan allocates (outputs, partials,
+    workspace, batch rows past B in a group of 16): forward and backward are finite and those
+    of the first run bit for bit."""
+    inp = core_case(300 + H, B, T, H)
+    first = None
+    for poisoned in (False, True):
+        x, out = _run_core(inp, dtype, cuda_device)
+        grads = [g.to(torch.bfloat16).float() for g in _core_grads(9, out)]
+        if poisoned:
+            # Blocks of both of the allocator's pools; what is freed here is handed out next.
+            junk = [torch.full((n,), float("nan"), device=cuda_device)
+                    for n in [1 << 16] * 64 + [1 << 22] * 24 + [1 << 26] * 4]
+            torch.cuda.synchronize()
+            del junk
+            x, out = _run_core(inp, dtype, cuda_device)
+        res = _hip_core_bwd(x, out, grads, dtype, cuda_device)
+        got = [t.clone() for t in (*out, *res)]
+        torch.cuda.synchronize()
+        assert all(bool(torch.isfinite(t).all()) for t in got)
+        if first is None:
+            first = got
+        else:
+            assert all(torch.equal(a, b) for a, b in zip(got, first))
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("B,T,H", [(2, 4, 1), (2, 5, 63), (3, 31, 65), (2, 63, 64), (1, 65, 130),
                                    (2, 127, 33), (2, 128, 15), (3, 129, 17), (1, 511, 64),
