@@ -26,6 +26,7 @@
 //
 // Bound by memory and, nearly as much, by the vector ALU (a step is about 56 instructions
 // forward and 91 backward): see the figures at the launchers.
+#include <algorithm>
 #include <type_traits>
 
 #include "../../include/dabsn_hip.h"
@@ -633,6 +634,16 @@ using namespace dabsn::longmem;
 
 constexpr int kBigRow = 1 << 24;  // see Rows
 
+constexpr int64_t kMaxChunks = 65536;  // longer sequences are refused: checked up to 2^17 steps
+
+// Batch rows lie in gridDim.y, which holds 65,535: larger batches (of few, narrow channels) run
+// as launches of that many rows each.
+constexpr int64_t kSlab = 65535;
+template <typename P>
+static P* row_ptr(P* p, int64_t b0, int64_t stride) {
+  return p ? p + b0 * stride : p;
+}
+
 // Chunks per wave. A workgroup of 64 channels walks T serially, so few channels leave most CUs
 // idle: up to kFew such workgroups a wave takes 4 chunks of 16 channels instead, 4 times the
 // workgroups and a quarter of the blocks (at accesses of 32 bytes, which so few channels can
@@ -664,26 +675,31 @@ static int long_fwd_impl(int B, int T, int H, int64_t ldx, const E* w, const E* 
     return DABSN_OK;
   }
   const int nseg = (T + CK - 1) / CK;
-  const dim3 grid(channel_tiles(B, T, H), B);
   const bool split = wave_chunks(B, T, H) == 4;
+  const int64_t n = static_cast<int64_t>(T) * H;
+  for (int64_t b0 = 0; b0 < B; b0 += kSlab) {
+    const dim3 grid(channel_tiles(B, T, H), static_cast<unsigned>(std::min(kSlab, B - b0)));
+    const int64_t r = b0 * H;
 #define DABSN_LONG(NW, G, BIG)                                                               \
   hipLaunchKernelGGL((long_fwd_kernel<E, NW, G, BIG>), grid, dim3(NW * LANES), 0, stream, T, H, ldx, \
-                     w, p, lg, L0, E0, R0, out, LF, EF, RF, keep)
-  if (H >= kBigRow)
-    DABSN_LONG(4, 1, true);
-  else if (split && nseg <= 16)
-    DABSN_LONG(4, 4, false);
-  else if (split)
-    DABSN_LONG(8, 4, false);
-  else if (nseg <= 1)
-    DABSN_LONG(1, 1, false);
-  else if (nseg <= 2)
-    DABSN_LONG(2, 1, false);
-  else if (nseg <= 4)
-    DABSN_LONG(4, 1, false);
-  else
-    DABSN_LONG(8, 1, false);
+                     w + b0 * ldx, p + b0 * ldx, lg, L0 + r, E0 + r, R0 + r, out + b0 * n, LF + r,  \
+                     EF + r, RF + r, row_ptr(keep, b0, 3ll * nseg * H))
+    if (H >= kBigRow)
+      DABSN_LONG(4, 1, true);
+    else if (split && nseg <= 16)
+      DABSN_LONG(4, 4, false);
+    else if (split)
+      DABSN_LONG(8, 4, false);
+    else if (nseg <= 1)
+      DABSN_LONG(1, 1, false);
+    else if (nseg <= 2)
+      DABSN_LONG(2, 1, false);
+    else if (nseg <= 4)
+      DABSN_LONG(4, 1, false);
+    else
+      DABSN_LONG(8, 1, false);
 #undef DABSN_LONG
+  }
   DABSN_HIP_CHECK(hipGetLastError());
   return DABSN_OK;
 }
@@ -694,24 +710,31 @@ static int long_bwd_impl(int B, int T, int H, int64_t ldx, const E* w, const E* 
                          const float* ckpt, const E* gout, const float* gLF, const float* gEF,
                          const float* gRF, E* gw, E* gp, int64_t ldo, float* gL0, float* gE0,
                          float* gR0, float* part, hipStream_t stream) {
-  const int nseg = (T + CK - 1) / CK;
-  const dim3 grid(channel_tiles(B, T, H), B);
+  const int nseg = (T + CK - 1) / CK, tiles = channel_tiles(B, T, H);
+  const int64_t n = static_cast<int64_t>(T) * H;
+  for (int64_t b0 = 0; b0 < B; b0 += kSlab) {
+    const dim3 grid(tiles, static_cast<unsigned>(std::min(kSlab, B - b0)));
+    const int64_t r = b0 * H;
 #define DABSN_LONG(NW, G, BIG)                                                                  \
   hipLaunchKernelGGL((long_bwd_kernel<E, ACC, NW, G, BIG>), grid, dim3(NW * LANES), 0, stream, T, H, \
-                     ldx, ldo, w, p, lg, ckpt, gout, gLF, gRF, gEF, gw, gp, gL0, gR0, gE0, part)
-  if (H >= kBigRow)
-    DABSN_LONG(4, 1, true);
-  else if (wave_chunks(B, T, H) == 4)
-    DABSN_LONG(4, 4, false);
-  else if (nseg <= 1)
-    DABSN_LONG(1, 1, false);
-  else if (nseg <= 2)
-    DABSN_LONG(2, 1, false);
-  else if (nseg <= 4 || static_cast<int64_t>(grid.x) * B > 256 || !is_bf16<E>::value)
-    DABSN_LONG(4, 1, false);
-  else if constexpr (is_bf16<E>::value)
-    DABSN_LONG(8, 1, false);
+                     ldx, ldo, w + b0 * ldx, p + b0 * ldx, lg, row_ptr(ckpt, b0, 3ll * nseg * H),     \
+                     row_ptr(gout, b0, n), row_ptr(gLF, b0, H), row_ptr(gRF, b0, H),                  \
+                     row_ptr(gEF, b0, H), row_ptr(gw, b0, ldo), row_ptr(gp, b0, ldo), gL0 + r, gR0 + r, \
+                     gE0 + r, part + 4 * b0 * tiles)
+    if (H >= kBigRow)
+      DABSN_LONG(4, 1, true);
+    else if (wave_chunks(B, T, H) == 4)
+      DABSN_LONG(4, 4, false);
+    else if (nseg <= 1)
+      DABSN_LONG(1, 1, false);
+    else if (nseg <= 2)
+      DABSN_LONG(2, 1, false);
+    else if (nseg <= 4 || static_cast<int64_t>(tiles) * B > 256 || !is_bf16<E>::value)
+      DABSN_LONG(4, 1, false);
+    else if constexpr (is_bf16<E>::value)
+      DABSN_LONG(8, 1, false);
 #undef DABSN_LONG
+  }
   DABSN_HIP_CHECK(hipGetLastError());
   return DABSN_OK;
 }
@@ -789,7 +812,7 @@ int dabsn_hip_long_fwd(int dtype, int64_t B, int64_t T, int64_t H, int64_t ldx, 
   (void)workspace;
   (void)workspace_bytes;
   for (int i = 0; i < 4; ++i) DABSN_REQUIRE(logits[i], "long scan: null logit %d", i);
-  DABSN_REQUIRE((T + CK - 1) / CK < 65536, "long scan: T too long");
+  DABSN_REQUIRE((T + CK - 1) / CK < kMaxChunks, "long scan: T too long");
   Logits lg{{logits[0], logits[1], logits[2], logits[3]}};
   if (dtype == kBF16)
     return long_fwd_impl<bf16>((int)B, (int)T, (int)H, lx, (const bf16*)w, (const bf16*)p, lg,
@@ -820,7 +843,7 @@ int dabsn_hip_long_bwd(int dtype, int64_t B, int64_t T, int64_t H, int64_t ldx, 
   (void)workspace;
   (void)workspace_bytes;
   for (int i = 0; i < 4; ++i) DABSN_REQUIRE(logits[i], "long scan backward: null logit %d", i);
-  DABSN_REQUIRE((T + CK - 1) / CK < 65536, "long scan backward: T too long");
+  DABSN_REQUIRE((T + CK - 1) / CK < kMaxChunks, "long scan backward: T too long");
   Logits lg{{logits[0], logits[1], logits[2], logits[3]}};
 #define DABSN_LONG_BWD(E, ACC)                                                                 \
   return long_bwd_impl<E, ACC>((int)B, (int)T, (int)H, lx, (const E*)w, (const E*)p, lg, ckpt,   \

@@ -398,6 +398,30 @@ def test_long_scan_block_edges(cuda_device, dtype, B, T, H):
     assert torch.equal(got[:, :, keep], out[0][:, :, keep])
 
 
+@pytest.mark.parametrize("T", [5, 70])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_long_scan_of_more_rows_than_a_grid_dimension_holds(cuda_device, dtype, T):
+    """70,001 batch rows: every row as in calls on the row blocks alone, bit for bit (rows are
+    independent), forward and backward; the logits' gradients, sums over all rows in another
+    order, to 1e-5."""
+    B, H, cut = 70001, 3, 30000
+    g = torch.Generator(device=cuda_device).manual_seed(T)
+    r = lambda *s: torch.randn(*s, device=cuda_device, generator=g)  # noqa: E731
+    w, p, go = r(B, T, H).to(dtype), r(B, T, H).sigmoid().to(dtype), r(B, T, H).to(dtype)
+    lg = [torch.tensor([v], device=cuda_device) for v in (2.2, 2.0, 2.4, 1.4)]
+    st, gf = [r(B, H) for _ in range(3)], [r(B, H) for _ in range(3)]
+    out = ops.long_scan_window(w, p, lg, *st)
+    res = ops.long_scan_backward_parts(w, p, lg, out[4], go, *gf)
+    logit_sum = torch.zeros(4, device=cuda_device, dtype=torch.float64)
+    for s in (slice(0, cut), slice(cut, B)):
+        o = ops.long_scan_window(w[s], p[s], lg, *[x[s] for x in st])
+        b = ops.long_scan_backward_parts(w[s], p[s], lg, o[4], go[s], *[x[s] for x in gf])
+        assert all(torch.equal(x[s], y) for x, y in zip(out, o))
+        assert all(torch.equal(x[s], y) for x, y in zip((*res[:2], *res[3]), (*b[:2], *b[3])))
+        logit_sum += b[2].double()
+    assert float((res[2].double() - logit_sum).norm()) <= 1e-5 * float(logit_sum.norm())
+
+
 @pytest.mark.parametrize("whole", [0, 1])
 @pytest.mark.parametrize("T", [1, 255, 256, 257, 3000, 16384])
 def test_bank_select_bit_exact(cuda_device, T, whole):
