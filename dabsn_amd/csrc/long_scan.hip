@@ -410,7 +410,8 @@ __global__ void __launch_bounds__(NT) long_fwd_single(int B, int T, int H, int64
 // ACC: gw += the gradient rounded to E, the sum formed in fp32 and rounded once (an add of
 // the rounded gradient into an existing gradient buffer).
 // The wave keeps 7 values per step (w and p of bf16 in one register): at most 256 registers,
-// 8 waves per CU; fp32 workgroups have 4 waves, which may use twice as many.
+// 8 waves per CU; the 4-wave workgroups of fp32 and of the 16-channel split (one per CU) may use
+// twice as many, and spill nothing (B=1, T=4096, H=64 bf16: 89 -> 80 us).
 template <typename E>
 struct Pair {  // w and p of one step
   E w, p;
@@ -434,9 +435,23 @@ struct Pair<bf16> {
   __device__ __forceinline__ void opaque_() { opaque(v); }
 };
 
+// The upstream gradient of one step and (KEEP) the value its write gradient is added to.
+template <typename E, bool KEEP>
+struct Grads {
+  E g;
+  __device__ __forceinline__ float up() const { return to_f(g); }
+  __device__ __forceinline__ void opaque_() { opaque(g); }
+};
+template <typename E>
+struct Grads<E, true> {
+  Pair<E> v;
+  __device__ __forceinline__ float up() const { return v.fp(); }
+  __device__ __forceinline__ void opaque_() { v.opaque_(); }
+};
+
 template <typename E, bool ACC, int NW, int G, bool BIG>
-__global__ void __launch_bounds__(NW* LANES, is_bf16<E>::value ? 2 : 1)
-    long_bwd_kernel(int T, int H, int64_t ldx, int64_t ldo, const E* __restrict__ w,
+__global__ void __launch_bounds__(NW* LANES, is_bf16<E>::value && G == 1 ? 2 : 1)
+    long_bwd_kernel(int T, int H, int64_t ldx, int64_t ldw, int64_t ldo, const E* __restrict__ w,
                     const E* __restrict__ p, Logits lg, const float* __restrict__ ckpt,
                     const E* __restrict__ gout, const float* __restrict__ gLF,
                     const float* __restrict__ gRF, const float* __restrict__ gEF,
@@ -458,7 +473,7 @@ __global__ void __launch_bounds__(NW* LANES, is_bf16<E>::value ? 2 : 1)
   E* wb = const_cast<E*>(w) + static_cast<size_t>(b) * ldx;
   E* pb = const_cast<E*>(p) + static_cast<size_t>(b) * ldx;
   E* gb = const_cast<E*>(gout) + static_cast<size_t>(b) * T * H;
-  E* gwb = gw + static_cast<size_t>(b) * ldo;
+  E* gwb = gw + static_cast<size_t>(b) * ldw;
   E* gpb = gp + static_cast<size_t>(b) * ldo;
   const int nseg = (T + CK - 1) / CK, nfull = T / CK, tail = T % CK;
   float t_er = 0.f, t_rd = 0.f, t_ret = 0.f, t_rs = 0.f;
@@ -474,13 +489,17 @@ __global__ void __launch_bounds__(NW* LANES, is_bf16<E>::value ? 2 : 1)
     const Rows<E, BIG> wr(wb + base, H, h, len, first), pr(pb + base, H, h, len, first),
         grow(gb + base, H, h, len, first), gwr(gwb + base, H, h, len, first),
         gpr(gpb + base, H, h, len, first);
+    constexpr bool KEEP = ACC && !(is_bf16<E>::value && G == 1);
     Pair<E> wp[CK];
-    E gr[CK];
+    Grads<E, KEEP> gr[CK];
 #pragma unroll
     for (int i = 0; i < CK; ++i) {
       const int j = full && !BIG ? i : min(i, max(len - 1, 0));
       wp[i].set(wr.load(j), pr.load(j));
-      gr[i] = grow.load(j);
+      if constexpr (KEEP)
+        gr[i].v.set(gwr.load(j), grow.load(j));
+      else
+        gr[i].g = grow.load(j);
     }
     __builtin_amdgcn_sched_barrier(0);
     const float* c = ckpt + (static_cast<size_t>(b) * nseg + (mine ? seg : 0)) * 3 * H;
@@ -495,7 +514,7 @@ __global__ void __launch_bounds__(NW* LANES, is_bf16<E>::value ? 2 : 1)
       for (int i = 0; i < CK; ++i) {
         wp[i].opaque_();
         opaque(R[i]);
-        opaque(gr[i]);
+        gr[i].opaque_();
       }
     };
     float r = Rs;
@@ -522,7 +541,7 @@ __global__ void __launch_bounds__(NW* LANES, is_bf16<E>::value ? 2 : 1)
     for (int i = CK - 1; i >= 0; --i)
         if (full || i < tail) {
           const float eff = retention(k, R[i]);
-          l = eff * (l + to_f(gr[i]));
+          l = eff * (l + gr[i].up());
           prod *= eff;
           fence(i);
         }
@@ -536,7 +555,7 @@ __global__ void __launch_bounds__(NW* LANES, is_bf16<E>::value ? 2 : 1)
 #pragma unroll
     for (int i = CK - 1; i >= 0; --i)
         if (full || i < tail) {
-          g[i] = l + to_f(gr[i]);
+          g[i] = l + gr[i].up();
           l = g[i] * retention(k, R[i]);
           a[i] = g[i] * a[i];
           r = fmaf(a[i], kap, r) * k.rd;
@@ -572,23 +591,39 @@ __global__ void __launch_bounds__(NW* LANES, is_bf16<E>::value ? 2 : 1)
           gpr.store(i, from_f<E>(dsal * pi));
           if (i % 4 == 0) __builtin_amdgcn_sched_barrier(0);
         }
-    E sv[ACC ? CK : 1];
-    if constexpr (ACC) {
+    // ACC: the values added to. With registers to spare (KEEP) they came with the inputs; else in
+    // groups of 8 rows, a group ahead of the stores of the one before it (all 32 at once spill).
+    constexpr int SG = 8;
+    constexpr bool LATE = ACC && !KEEP;
+    E sv[2][SG];
+    auto load_into = [&](int g0, E(&dst)[SG]) {
+      if constexpr (LATE) {
 #pragma unroll
-      for (int i = 0; i < CK; ++i) sv[i] = gwr.load(full && !BIG ? i : min(i, max(len - 1, 0)));
-    }
+        for (int i = 0; i < SG; ++i)
+          dst[i] = gwr.load(full && !BIG ? g0 + i : min(g0 + i, max(len - 1, 0)));
+      }
+    };
+    load_into(CK - SG, sv[0]);
     se[idx][lc] = e;
     __syncthreads();
     e = enter<NC, LC, true>(gEc, se, nullptr, er_pow, idx, lc, live);
 #pragma unroll
-    for (int i = CK - 1; i >= 0; --i)
+    for (int q = 0; q < CK / SG; ++q) {
+      const int g0 = CK - SG * (q + 1);
+      if (LATE && g0 > 0) load_into(g0 - SG, sv[(q + 1) & 1]);
+      if constexpr (LATE) __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int i = g0 + SG - 1; i >= g0; --i)
         if (full || i < tail) {
           float v = fmaf(1.0f - k.er, e, g[i]);
-          if constexpr (ACC) v = to_f(sv[i]) + round_to<E>(v);
+          if constexpr (KEEP) v = gr[i].v.fw() + round_to<E>(v);
+          if constexpr (LATE) v = to_f(sv[q & 1][i - g0]) + round_to<E>(v);
           d_er = fmaf(-e, diff[i], d_er);
           e = fmaf(k.er, e, -pe[i]);
           gwr.store(i, from_f<E>(v));
         }
+      if constexpr (LATE) __builtin_amdgcn_sched_barrier(0);
+    }
     t_er += mine ? d_er : 0.0f;
     t_rd += mine ? d_rd : 0.0f;
     t_ret += mine ? d_ret : 0.0f;
@@ -619,6 +654,16 @@ __global__ void __launch_bounds__(NW* LANES, is_bf16<E>::value ? 2 : 1)
   }
 }
 
+// gw[b][i] += g[b][i], the sum formed in fp32 and rounded once (see the backward's launcher).
+template <typename E>
+__global__ void __launch_bounds__(256) long_add_kernel(int64_t n, int64_t ldw, const E* __restrict__ g,
+                                                       E* __restrict__ gw) {
+  const int64_t i = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
+  if (i >= n) return;
+  E* o = gw + blockIdx.y * ldw + i;
+  *o = from_f<E>(to_f(*o) + to_f(g[blockIdx.y * n + i]));
+}
+
 static int grid_for(int64_t B, int64_t H) { return static_cast<int>((B * H + NT - 1) / NT); }
 
 }  // namespace longmem
@@ -647,9 +692,9 @@ static P* row_ptr(P* p, int64_t b0, int64_t stride) {
 // Chunks per wave. A workgroup of 64 channels walks T serially, so few channels leave most CUs
 // idle: up to kFew such workgroups a wave takes 4 chunks of 16 channels instead, 4 times the
 // workgroups and a quarter of the blocks (at accesses of 32 bytes, which so few channels can
-// afford). Backward, bf16: B=1, T=4096, H=64 takes 184 us with 64 channels and 85 with 16 (the
-// earlier kernels, parallel over all chunks of T: 78); B=8, T=2573, H=400 (56 workgroups) 134
-// and 99 (117); B=32, T=3200, H=256 (128 workgroups) 175 and 187 (217).
+// afford). Backward, bf16: B=1, T=4096, H=64 takes 184 us with 64 channels and 80 with 16 (the
+// earlier kernels, parallel over all chunks of T: 74; forward 140 against 68); B=8, T=2573, H=400
+// (56 workgroups) 134 and 86 (114); B=32, T=3200, H=256 (128 workgroups) 174 and 187 (215).
 constexpr int64_t kFew = 64;
 static int wave_chunks(int64_t B, int64_t T, int64_t H) {
   return B * ((H + LANES - 1) / LANES) <= kFew && T >= 4 * CK ? 4 : 1;
@@ -704,26 +749,44 @@ static int long_fwd_impl(int B, int T, int H, int64_t ldx, const E* w, const E* 
   return DABSN_OK;
 }
 
-// B=16, T=4096, H=2048 bf16: 891 -> 482 us (1.39 GB: 2.9 TB/s).
+// B=16, T=4096, H=2048 bf16: 891 -> 425 us (1.39 GB: 3.3 TB/s); accumulating, on half of the CUs
+// and T=768, 307 -> 177.
+//
+// ACC with 16-channel tiles: a 128-byte line of gw then belongs to several workgroups, on several
+// XCDs, and reading lines that another XCD writes stalls each block (B=1, T=4096, H=64 bf16: 235
+// us against 80 without ACC). So the split scan writes its gradient to the workspace `ws`, whole,
+// and another kernel adds it.
 template <typename E, bool ACC>
 static int long_bwd_impl(int B, int T, int H, int64_t ldx, const E* w, const E* p, Logits lg,
                          const float* ckpt, const E* gout, const float* gLF, const float* gEF,
-                         const float* gRF, E* gw, E* gp, int64_t ldo, float* gL0, float* gE0,
-                         float* gR0, float* part, hipStream_t stream) {
-  const int nseg = (T + CK - 1) / CK, tiles = channel_tiles(B, T, H);
+                         const float* gRF, E* gw, int64_t ldw, E* gp, int64_t ldo, float* gL0,
+                         float* gE0, float* gR0, float* part, E* ws, hipStream_t stream) {
+  const bool split = wave_chunks(B, T, H) == 4;
   const int64_t n = static_cast<int64_t>(T) * H;
+  if constexpr (ACC) {
+    if (split && ws) {
+      const int rc = long_bwd_impl<E, false>(B, T, H, ldx, w, p, lg, ckpt, gout, gLF, gEF, gRF, ws, n,
+                                             gp, ldo, gL0, gE0, gR0, part, nullptr, stream);
+      if (rc != DABSN_OK) return rc;
+      hipLaunchKernelGGL(long_add_kernel<E>, dim3(static_cast<unsigned>((n + 255) / 256), B), dim3(256),
+                         0, stream, n, ldw, ws, gw);
+      DABSN_HIP_CHECK(hipGetLastError());
+      return DABSN_OK;
+    }
+  }
+  const int nseg = (T + CK - 1) / CK, tiles = channel_tiles(B, T, H);
   for (int64_t b0 = 0; b0 < B; b0 += kSlab) {
     const dim3 grid(tiles, static_cast<unsigned>(std::min(kSlab, B - b0)));
     const int64_t r = b0 * H;
 #define DABSN_LONG(NW, G, BIG)                                                                  \
   hipLaunchKernelGGL((long_bwd_kernel<E, ACC, NW, G, BIG>), grid, dim3(NW * LANES), 0, stream, T, H, \
-                     ldx, ldo, w + b0 * ldx, p + b0 * ldx, lg, row_ptr(ckpt, b0, 3ll * nseg * H),     \
+                     ldx, ldw, ldo, w + b0 * ldx, p + b0 * ldx, lg, row_ptr(ckpt, b0, 3ll * nseg * H), \
                      row_ptr(gout, b0, n), row_ptr(gLF, b0, H), row_ptr(gRF, b0, H),                  \
-                     row_ptr(gEF, b0, H), row_ptr(gw, b0, ldo), row_ptr(gp, b0, ldo), gL0 + r, gR0 + r, \
+                     row_ptr(gEF, b0, H), row_ptr(gw, b0, ldw), row_ptr(gp, b0, ldo), gL0 + r, gR0 + r, \
                      gE0 + r, part + 4 * b0 * tiles)
     if (H >= kBigRow)
       DABSN_LONG(4, 1, true);
-    else if (wave_chunks(B, T, H) == 4)
+    else if (split)
       DABSN_LONG(4, 4, false);
     else if (nseg <= 1)
       DABSN_LONG(1, 1, false);
@@ -786,8 +849,11 @@ int dabsn_hip_linrec_bwd(int dtype, int64_t B, int64_t T, int64_t H, const void*
   return DABSN_OK;
 }
 
-size_t dabsn_hip_long_workspace_bytes(int64_t, int64_t, int64_t, int) {
-  return 0;  // the chunk ends stay in LDS
+// Only the accumulating backward (bit 2 of `backward`) of few channels keeps anything outside its
+// registers and LDS: the gradient it adds.
+size_t dabsn_hip_long_workspace_bytes(int64_t B, int64_t T, int64_t H, int backward) {
+  if (!(backward & 2) || B <= 0 || T <= 0 || H <= 0 || wave_chunks(B, T, H) != 4) return 0;
+  return static_cast<size_t>(B) * T * H * sizeof(float);
 }
 
 // Batch stride of [B, T, H] operands: ldx elements (0: T H, the contiguous layout); at least
@@ -840,15 +906,14 @@ int dabsn_hip_long_bwd(int dtype, int64_t B, int64_t T, int64_t H, int64_t ldx, 
   DABSN_REQUIRE(w && p && logits && (ckpt || T == 0) && (gout || T == 0) && gL0 && gE0 && gR0 &&
                     part_logit && ((gw && gp) || T == 0),
                 "long scan backward: null pointer");
-  (void)workspace;
-  (void)workspace_bytes;
   for (int i = 0; i < 4; ++i) DABSN_REQUIRE(logits[i], "long scan backward: null logit %d", i);
   DABSN_REQUIRE((T + CK - 1) / CK < kMaxChunks, "long scan backward: T too long");
   Logits lg{{logits[0], logits[1], logits[2], logits[3]}};
 #define DABSN_LONG_BWD(E, ACC)                                                                 \
   return long_bwd_impl<E, ACC>((int)B, (int)T, (int)H, lx, (const E*)w, (const E*)p, lg, ckpt,   \
-                               (const E*)gout, gLF, gEF, gRF, (E*)gw, (E*)gp, lo, gL0, gE0, gR0, \
-                               part_logit, stream)
+                               (const E*)gout, gLF, gEF, gRF, (E*)gw, lo, (E*)gp, lo, gL0, gE0, \
+                               gR0, part_logit, workspace && workspace_bytes >= B * T * H * sizeof(E) \
+                               ? static_cast<E*>(workspace) : nullptr, stream)
   if (dtype == kBF16) {
     if (gw_accumulate) DABSN_LONG_BWD(bf16, true);
     DABSN_LONG_BWD(bf16, false);

@@ -1342,7 +1342,7 @@ def long_scan_backward_parts(
     nparts = lib.dabsn_hip_long_partials(B, T, H)
     part = torch.empty((max(nparts, 1), 4), device=w.device, dtype=torch.float32)
     part[nparts:].zero_()
-    nbytes = lib.dabsn_hip_long_workspace_bytes(B, T, H, 1)
+    nbytes = lib.dabsn_hip_long_workspace_bytes(B, T, H, 1 | 2 * acc)
     ws = torch.empty(max(nbytes, 4), dtype=torch.uint8, device=w.device)
     tk = KernelTimer.begin("long_scan_bwd", w)
     st = checkpoint.float().contiguous()

@@ -180,7 +180,8 @@ int dabsn_hip_linrec_bwd(int dtype, int64_t B, int64_t T, int64_t H, const void*
  * read.py:625-636). logits[4] point at fp32 scalars (logit_expect_retain,
  * logit_retention_decay, logit_retain, logit_retention_strength). State L0/E0/R0 [B,H]
  * fp32 in, LF/EF/RF out. Both directions are chunked over time (chunks of DABSN_LONG_CKPT
- * steps) and need dabsn_hip_long_workspace_bytes() bytes of workspace (0: none). `ckpt` (may be NULL)
+ * steps). dabsn_hip_long_workspace_bytes(): `backward` 0, 1, or 3 for a backward with
+ * gw_accumulate; all but the last, of few channels, are 0. `ckpt` (may be NULL)
  * receives the checkpoint the backward replays each chunk from: the fp32 states entering
  * every chunk, [B][ceil(T / DABSN_LONG_CKPT)][3][H] = (L, E, R). `ldx`: elements between
  * the batch rows of w and p (0: T H, contiguous; otherwise >= T H, e.g. a time window of
@@ -198,7 +199,7 @@ int dabsn_hip_long_fwd(int dtype, int64_t B, int64_t T, int64_t H, int64_t ldx, 
  * and part_logit [nblocks][4] with nblocks = dabsn_hip_long_partials(B, T, H): per-block
  * partial sums of the gradient w.r.t. the four logits. gw_accumulate != 0: gw receives
  * gw + (the gradient rounded to dtype), summed in fp32 and rounded once -- an add into an
- * existing gradient buffer. */
+ * existing gradient buffer. The workspace may be NULL (a slower route, the same bits). */
 int64_t dabsn_hip_long_partials(int64_t B, int64_t T, int64_t H);
 int dabsn_hip_long_bwd(int dtype, int64_t B, int64_t T, int64_t H, int64_t ldx, const void* w,
                        const void* p, const float* const* logits, const float* ckpt,

@@ -398,6 +398,34 @@ def test_long_scan_block_edges(cuda_device, dtype, B, T, H):
     assert torch.equal(got[:, :, keep], out[0][:, :, keep])
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("B,T,H", [(2, 127, 70), (2, 128, 70), (64, 128, 64), (65, 128, 64)])
+def test_long_scan_backward_accumulates_with_and_without_workspace(cuda_device, dtype, B, T, H):
+    """Few channels add their write gradient from a workspace, or in the scan where the caller
+    gives none: both are the plain gradient added, bit for bit."""
+    g = torch.Generator(device=cuda_device).manual_seed(B + T)
+    r = lambda *s: torch.randn(*s, device=cuda_device, generator=g)  # noqa: E731
+    w, p, go = r(B, T, H).to(dtype), r(B, T, H).sigmoid().to(dtype), r(B, T, H).to(dtype)
+    lg = [torch.tensor([v], device=cuda_device) for v in (2.2, 2.0, 2.4, 1.4)]
+    ckpt = ops.long_scan_window(w, p, lg, *[r(B, H) for _ in range(3)])[4]
+    plain = ops.long_scan_backward_parts(w, p, lg, ckpt, go, None, None, None)
+    base = r(B, T, H).to(dtype)
+    lib, P = ops._lib.load(), lambda t: t.data_ptr()
+    assert (lib.dabsn_hip_long_workspace_bytes(B, T, H, 3) > 0) == (B <= 64 and T >= 128)
+    assert lib.dabsn_hip_long_workspace_bytes(B, T, H, 1) == 0
+    gw, gp = base.clone(), torch.empty_like(base)
+    got = ops.long_scan_backward_parts(w, p, lg, ckpt, go, None, None, None, gw, gp)
+    part = torch.empty(lib.dabsn_hip_long_partials(B, T, H), 4, device=cuda_device)
+    bare = [base.clone(), torch.empty_like(base), *[torch.empty(B, H, device=cuda_device) for _ in range(3)]]
+    ops._lib.check(lib.dabsn_hip_long_bwd(
+        ops._code(dtype), B, T, H, 0, P(w), P(p), ops._lib.PTR4(*[P(x) for x in lg]), P(ckpt), P(go),
+        None, None, None, P(bare[0]), P(bare[1]), 0, 1, *[P(x) for x in bare[2:]], P(part), None, 0,
+        ops._stream(w)), "long scan backward")
+    for a, b, c in zip((gw, gp, got[2], *got[3]), (bare[0], bare[1], part.t().contiguous().sum(1), *bare[2:]),
+                       (base + plain[0], plain[1], plain[2], *plain[3])):
+        assert torch.equal(a, c) and torch.equal(b, c)
+
+
 @pytest.mark.parametrize("T", [5, 70])
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 def test_long_scan_of_more_rows_than_a_grid_dimension_holds(cuda_device, dtype, T):
