@@ -7,9 +7,9 @@ one readout GEMM (hipBLASLt through ``F.linear``), and one HIP row kernel
 logits once in their own dtype instead of an fp32 copy plus logsumexp / gather kernels.
 The backward recomputes each chunk's logits, forms (softmax - onehot) * scale in one row
 kernel (``ops.ce_rows_backward``, reusing the forward's logsumexp), and runs the two
-gradient GEMMs in fp32 as the reference does (loss.py:95-137); for bf16 readouts the fp32
-rows are split into three bf16 planes that hold all of their bits, and the GEMMs are bf16
-with fp32 accumulation (``ops.linear_ce_backward_bf16``).
+gradient GEMMs in fp32 as the reference does (loss.py:95-137); for large bf16 readouts the
+fp32 rows are split into three bf16 planes that hold all of their bits, and the GEMMs are
+bf16 with fp32 accumulation (``ops.linear_ce_backward_bf16``).
 
 Same API, defaults and environment switch as the reference: ``DABSN_LOSS_CHUNK_SCORES``
 sets the element budget (default 2**24), ``off`` forces ``F.cross_entropy`` on the full
@@ -18,6 +18,7 @@ logits. Inputs must be device tensors (fp32 or bf16); the loss is fp32.
 
 from __future__ import annotations
 
+import contextlib
 import os
 
 import torch
@@ -67,6 +68,20 @@ def _rows(parts: list[Tensor], like: Tensor) -> Tensor:
     return parts[0] if len(parts) == 1 else torch.cat(parts)
 
 
+def _split_pays(n: int, vocab: int, width: int) -> bool:
+    """Whether a bf16 readout's gradient products run over the three bf16 planes of the
+    gradient (``ops.linear_ce_backward_bf16``) or in fp32 on fp32 copies. The planes save most
+    of the fp32 products' time, in proportion to vocab * width a row; they cost three fp32 rows
+    of the hidden width a row (as much as the products of 900 words save), products that sum
+    over three times as many rows into few tiles where the weight is small, and launches.
+    Backward on MI355X, fp32 -> planes in us, N=16384 if not said: V=60 H=2048 359 -> 647, V=768
+    996 -> 1305, V=1024 H=1024 714 -> 807, V=1300 H=800 (whole pass) 1285 -> 1405, V=1500 H=700
+    914 -> 940, V=2048 H=256 (N=8192) 259 -> 328; V=1501 H=1023 1497 -> 1216, V=2000 H=512 892
+    -> 778, V=4000 H=256 1177 -> 932. Few rows: N=1024 V=2048 H=1024 182 -> 189, N=256 V=32000
+    H=64 207 -> 256; N=2048 V=32000 H=64 884 -> 840, N=256 V=32000 H=512 519 -> 286."""
+    return (vocab - 900) * width >= 500_000 and n * vocab * width >= 3_000_000_000
+
+
 class ChunkedLinearCrossEntropy(torch.autograd.Function):
     """Fused readout + mean cross-entropy that never holds more than [chunk, V] logits.
     Forward saves hidden, weight, bias, targets and the rows' logsumexp (N floats)."""
@@ -77,9 +92,9 @@ class ChunkedLinearCrossEntropy(torch.autograd.Function):
         acc = _accum_dtype(hidden.dtype)
         n = int(hidden.shape[0])
         lses, nlls = [], []
-        # On the device the chunks share one error word, read after the last of them.
-        word = (torch.zeros(1, device=hidden.device, dtype=torch.int32) if hidden.is_cuda
-                else None)
+        # On the device several chunks share one error word, read after the last of them.
+        word = (torch.zeros(1, device=hidden.device, dtype=torch.int32)
+                if hidden.is_cuda and n > chunk_rows else None)
         for s, e in _spans(n, chunk_rows):
             logits = F.linear(hidden[s:e], weight, bias)
             if word is None:
@@ -101,11 +116,15 @@ class ChunkedLinearCrossEntropy(torch.autograd.Function):
         hidden, weight, bias, targets, denom, lse = ctx.saved_tensors
         acc = ctx.acc
         scale = (grad_output / denom).to(torch.float32).reshape(1)
-        if hidden.is_cuda and hidden.dtype == weight.dtype == torch.bfloat16 and (
-                bias is None or bias.dtype == torch.bfloat16):
+        bf16 = hidden.is_cuda and hidden.dtype == weight.dtype == torch.bfloat16 and (
+            bias is None or bias.dtype == torch.bfloat16)
+        if bf16 and _split_pays(int(hidden.shape[0]), *(int(d) for d in weight.shape)):
             gh, gw, gb = ops.linear_ce_backward_bf16(hidden, weight, bias, targets, lse, scale,
                                                      ctx.chunk_rows, ctx.ignore_index)
             return (gh, gw, None if bias is None else gb.to(bias.dtype), None, None, None)
+        # A backward inside autocast would round the fp32 operands to 16 bits, which the split
+        # products of larger bf16 calls do not.
+        fp32_products = bf16 and torch.is_autocast_enabled("cuda")
         weight_acc = weight.to(acc)
         grad_hidden = torch.empty_like(hidden)
         grad_weight = torch.zeros_like(weight, dtype=acc)
@@ -114,8 +133,10 @@ class ChunkedLinearCrossEntropy(torch.autograd.Function):
             hid = hidden[s:e]
             logits = F.linear(hid, weight, bias)
             d = ops.ce_rows_backward(logits, targets[s:e], ctx.ignore_index, lse[s:e], scale)
-            grad_hidden[s:e] = torch.mm(d, weight_acc).to(hidden.dtype)
-            grad_weight.addmm_(d.t(), hid.to(acc))  # accumulated inside the GEMM
+            with (torch.autocast("cuda", enabled=False) if fp32_products
+                  else contextlib.nullcontext()):
+                grad_hidden[s:e] = torch.mm(d, weight_acc).to(hidden.dtype)
+                grad_weight.addmm_(d.t(), hid.to(acc))  # accumulated inside the GEMM
             if grad_bias is not None:
                 grad_bias += d.sum(dim=0)
         grad_weight = grad_weight.to(weight.dtype)

@@ -202,6 +202,59 @@ def test_bf16_readout_gradients_match_fp64(cuda_device, N, V, H, budget, bias):
         assert all(a is None or float(a.grad.float().abs().max()) == 0 for a in leaves)
 
 
+def test_the_split_products_run_where_they_pay():
+    """Small vocabularies, small weights and small calls keep the fp32 products."""
+    for n, v, h in [(16384, 60, 64), (16384, 60, 2048), (16384, 400, 2048), (16384, 1024, 1024),
+                    (8192, 2048, 256), (16384, 1300, 800), (256, 32000, 64), (300, 5001, 77), (0, 32000, 2048)]:
+        assert not L._split_pays(n, v, h)
+    for n, v, h in [(8192, 32000, 2048), (256, 32000, 2048), (6250, 32000, 64), (16384, 12000, 1024)]:
+        assert L._split_pays(n, v, h)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("N,V,H,chunk,bias", [(1, 5, 3, 1, True), (70, 33, 48, 16, True),
+                                              (64, 129, 96, 16, False), (300, 1000, 200, 40, True),
+                                              (513, 4099, 73, 63, True), (40, 70, 6, 40, True)])
+def test_split_products_match_the_fp32_ones(cuda_device, N, V, H, chunk, bias):
+    """Both routes of the bf16 readout's backward at sizes of either: one chunk, chunks in a
+    group, groups with a shorter last one, odd vocabularies and widths. Both products sum the
+    same exact terms in fp32 (some 1e-6 apart) and round once to bf16: a value near the middle
+    of two bf16 values rounds to either, 2^-8 of itself, so 2^-8 of the value."""
+    from dabsn_amd.kernels import ops
+
+    h, w, b, t = _case(N + V, 1, N, H, V, bias=bias, dtype=torch.bfloat16)
+    h, t = h.reshape(N, H).to(cuda_device), t.reshape(N).to(cuda_device)
+    w, b = w.to(cuda_device), None if b is None else b.to(cuda_device)
+    t[::7] = -100
+    lse, _ = ops.ce_rows(torch.nn.functional.linear(h, w, b), t, -100)
+    scale = torch.tensor([0.37], device=cuda_device)
+    gh, gw, gb = ops.linear_ce_backward_bf16(h, w, b, t, lse, scale, chunk, -100)
+    d = torch.cat([ops.ce_rows_backward(torch.nn.functional.linear(h[s:s + chunk], w, b),
+                                        t[s:s + chunk], -100, lse[s:s + chunk], scale)
+                   for s in range(0, N, chunk)]).double()
+    for got, want in ((gh, d @ w.double()), (gw, d.t() @ h.double())):
+        err = (got.double() - want).abs()
+        assert bool((err <= 2.0 ** -8 * want.abs() + 1e-6 * want.abs().max()).all())
+        assert float(err.norm()) <= 2.0 ** -8 * float(want.norm())
+    assert gb.numel() == (V if bias else 0)
+    if bias:
+        assert float((gb.double() - d.sum(0)).abs().max()) <= N * 2.0 ** -24
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("N,V,H", [(50, 100, 64), (1500, 2048, 1024)])
+def test_bf16_readout_backward_inside_autocast_keeps_fp32_products(cuda_device, N, V, H):
+    """The gradients of a backward call inside a bf16 autocast region are those of one outside."""
+    h, w, b, t = _case(N, 1, N, H, V, dtype=torch.bfloat16)
+    grads = []
+    for inside in (False, True):
+        leaves = [x.to(cuda_device).requires_grad_(True) for x in (h, w, b)]
+        with torch.autocast("cuda", torch.bfloat16, enabled=inside):
+            L.chunked_linear_cross_entropy(*leaves, t.to(cuda_device)).backward()
+        grads.append([x.grad for x in leaves])
+    assert all(torch.equal(x, y) for x, y in zip(*grads))
+
+
 @pytest.mark.gpu
 def test_bf16_readout_reports_a_bad_target_in_any_chunk(cuda_device):
     h, w, b, t = _case(9, 1, 40, 16, 30, dtype=torch.bfloat16)
