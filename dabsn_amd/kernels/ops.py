@@ -1047,8 +1047,13 @@ def linear_ce_backward_bf16(hidden: Tensor, weight: Tensor, bias: Optional[Tenso
     grad_bias = torch.zeros(V if bias is not None else 0, device=dev, dtype=f32)
     if N == 0:
         return grad_hidden, torch.zeros_like(weight), grad_bias
-    # Planes of 6 rows V bytes against 4 V H of the fp32 weight copy.
-    chunk = max(1, min(int(chunk_rows), N))
+    # Planes of 6 rows V bytes against 4 V H of the fp32 weight copy. A small vocabulary's chunks
+    # are long, and the products' fp32 rows and the three copies of the hidden rows (18 H bytes
+    # a row) would outgrow everything else: they stay within that copy or 512 MB (N=65536
+    # V=1200 H=4096: 2415 MB beside the inputs without this bound and the releases below, 988
+    # with them, 1101 with fp32 products).
+    fit = max(4 * V * H, 1 << 29) // (18 * H)
+    chunk = max(1, min(int(chunk_rows), N, fit))
     group = min(N, chunk * max(1, (2 * H // 3) // chunk))
     ldp = -(-V // 8) * 8
     planes = torch.empty((3, group, ldp), device=dev, dtype=torch.bfloat16)
@@ -1080,11 +1085,13 @@ def linear_ce_backward_bf16(hidden: Tensor, weight: Tensor, bias: Optional[Tenso
         gh = torch.mm(d, weight, out_dtype=f32)
         _lib.check(lib.dabsn_hip_ce_join((g1 - g0) * H, _p(gh), _p(grad_hidden[g0:g1]),
                                          _stream(gh)), "cross entropy backward")
+        del gh  # ahead of what the weight gradient and the next group allocate
         rows3 = torch.cat((rows, rows, rows))
         if grad_weight is None:
             grad_weight = torch.mm(d.t(), rows3, out_dtype=f32)
         else:
             torch.addmm(grad_weight, d.t(), rows3, out_dtype=f32, out=grad_weight)
+        del rows3
         if part is not None:
             _lib.check(lib.dabsn_hip_ce_bias(used, V, _p(part), int(g0 > 0), _p(grad_bias),
                                              _stream(part)), "cross entropy backward")

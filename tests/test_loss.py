@@ -242,6 +242,26 @@ def test_split_products_match_the_fp32_ones(cuda_device, N, V, H, chunk, bias):
 
 
 @pytest.mark.gpu
+def test_split_products_bound_their_memory(cuda_device):
+    """One chunk of many rows against few words: the products' copies (18 H bytes a row, 1.2 GB
+    for these rows at once) stay within 512 MB beside the gradients (151 MB), the planes and
+    logits (8 V bytes a row of a group) and the partials."""
+    from dabsn_amd.kernels import ops
+
+    N, V, H = 16384, 1024, 4096
+    h = torch.randn(N, H, device=cuda_device).to(torch.bfloat16)
+    w = torch.randn(V, H, device=cuda_device).to(torch.bfloat16)
+    t = torch.randint(0, V, (N,), device=cuda_device)
+    lse, scale = torch.zeros(N, device=cuda_device), torch.tensor([1e-9], device=cuda_device)
+    torch.cuda.synchronize()
+    torch.cuda.reset_peak_memory_stats()
+    base = torch.cuda.memory_allocated()
+    ops.linear_ce_backward_bf16(h, w, None, t, lse, scale, N, -100)
+    torch.cuda.synchronize()
+    assert torch.cuda.max_memory_allocated() - base <= (512 << 20) + (192 << 20)
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("N,V,H", [(50, 100, 64), (1500, 2048, 1024)])
 def test_bf16_readout_backward_inside_autocast_keeps_fp32_products(cuda_device, N, V, H):
     """The gradients of a backward call inside a bf16 autocast region are those of one outside."""
