@@ -250,8 +250,8 @@ __global__ void __launch_bounds__(256) perm_reduce_kernel(int64_t BT, int H, int
 //
 // Bound by the chunk's serial chain: the products (8 NT MFMAs of 32 cycles a wave, 22 NT + 8
 // backward), two barriers and the solve, about 1.6 us a chunk forward and 3.5 us backward at
-// H = 256. B = 16, T = 1024, H = 256, step by step -> in chunks: forward 576 -> 108 us with G,
-// backward 2410 -> 402 us; error against 64 bits 5.1e-7 -> 4.5e-7 at worst there, and over
+// H = 256. B = 16, T = 1024, H = 256, step by step -> in chunks: forward 576 -> 98 us with G,
+// backward 2410 -> 393 us; error against 64 bits 5.1e-7 -> 4.5e-7 at worst there, and over
 // H = 32..512, T = 60..1024 between 0.6 and 1.3 times the walk's, all below 5e-7.
 namespace chunked {
 
@@ -329,17 +329,11 @@ __device__ __forceinline__ f32x4 mask_k4(f32x4 v, int T, int H, int t, int c) {
   return v;
 }
 
-// G [B][chunks][16][16] of every chunk: one wave per chunk. With the k index permuted as
-// above the same registers are both operands.
+// One chunk's G (steps t0 ..) by one wave: lane's entries [4 (lane / 16) + i][lane % 16]. With the
+// k index permuted as above the same registers are both operands.
 template <bool VEC>
-__global__ void __launch_bounds__(NTH) gram_kernel(int T, int H, int nchunk, int64_t total,
-                                                   const float* __restrict__ k,
-                                                   float* __restrict__ gram) {
-  const int64_t id = static_cast<int64_t>(blockIdx.x) * (NTH / 64) + (threadIdx.x >> 6);
-  if (id >= total) return;  // whole waves
-  const int lane = threadIdx.x & 63;
-  const float* kb = k + static_cast<size_t>(id / nchunk) * T * H;
-  const int t = static_cast<int>(id % nchunk) * C + (lane & 15);
+__device__ __forceinline__ f32x4 gram_tile(const float* __restrict__ kb, int T, int H, int t0, int lane) {
+  const int t = t0 + (lane & 15);
   f32x4 a0 = {0.f, 0.f, 0.f, 0.f}, a1 = a0;
   for (int c = 4 * (lane >> 4); c < H + 4 * (lane >> 4); c += 32) {
     const f32x4 x = mask_k4(load_k4<VEC>(kb, T, H, t, c), T, H, t, c);
@@ -350,10 +344,50 @@ __global__ void __launch_bounds__(NTH) gram_kernel(int T, int H, int nchunk, int
       a1 = mma(y[i], y[i], a1);
     }
   }
-  a0 = a0 + a1;
-#pragma unroll
-  for (int i = 0; i < 4; ++i) gram[id * (C * C) + (4 * (lane >> 4) + i) * C + (lane & 15)] = a0[i];
+  return a0 + a1;
 }
+
+// G [B][chunks][16][16] of every chunk: one wave per chunk. Short scans of short keys have every
+// workgroup form its own in LDS instead (the same bits), which takes a launch and an allocation
+// out of each direction. us forward / backward on the device, with the kernel -> in LDS: B=1 T=16
+// H=32 6.0 / 12.8 -> 3.6 / 7.2 (the walk per step 5.2 / 25.5), B=16 T=64 H=256 12.5 / 39.2 -> 11.0
+// / 33.5, B=64 T=128 H=64 11.3 / 31.6 -> 10.0 / 27.5; but, every row block forming the same G,
+// B=64 T=128 H=256 40.8 / 182 -> 52.3 / 179, B=64 T=64 H=512 69.8 / 398 -> 96.5 / 465 and, past
+// the 2,048 row blocks that hide it in their launch, B=256 T=64 H=256 70.8 / 368 -> 90.5 / 382.
+constexpr int kShort = 8;
+static bool brief(int64_t B, int64_t T, int64_t H) {
+  return ((T <= kShort * C && H <= 128) || (T <= kShort / 2 * C && H <= 256)) && B * H <= 2048 * RB;
+}
+template <bool VEC>
+__global__ void __launch_bounds__(NTH) gram_kernel(int T, int H, int nchunk, int64_t total,
+                                                   const float* __restrict__ k,
+                                                   float* __restrict__ gram) {
+  const int64_t id = static_cast<int64_t>(blockIdx.x) * (NTH / 64) + (threadIdx.x >> 6);
+  if (id >= total) return;  // whole waves
+  const int lane = threadIdx.x & 63;
+  const f32x4 g = gram_tile<VEC>(k + static_cast<size_t>(id / nchunk) * T * H, T, H,
+                                 static_cast<int>(id % nchunk) * C, lane);
+#pragma unroll
+  for (int i = 0; i < 4; ++i) gram[id * (C * C) + (4 * (lane >> 4) + i) * C + (lane & 15)] = g[i];
+}
+
+// G of a short scan in LDS (SHORT), or row t of it in the workspace.
+template <int NT, bool SHORT>
+struct Gram {
+  float g[!SHORT ? 1 : NT <= 2 ? kShort : kShort / 2][C][C];
+  template <bool VEC>
+  __device__ __forceinline__ void fill(const float* __restrict__ kb, int T, int H, int nchunk) {
+    if constexpr (SHORT) {
+      const int lane = threadIdx.x & 63;
+      for (int n = threadIdx.x >> 6; n < nchunk; n += NTH / 64) {
+        const f32x4 v = gram_tile<VEC>(kb, T, H, n * C, lane);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) g[n][4 * (lane >> 4) + i][lane & 15] = v[i];
+      }
+      __syncthreads();
+    }
+  }
+};
 
 // A chunk's K rows in registers (one chunk ahead) and in LDS.
 template <int NT, bool VEC>
@@ -398,9 +432,16 @@ __device__ __forceinline__ void partial(const float (*kl)[Geo<NT>::LS], const f3
 struct StepIn {
   float x, beta, f;  // v (forward) or g and v - r (backward)
   f32x4 g[4];        // row t of G
-  __device__ __forceinline__ void load_row(const float* __restrict__ p) {
+  template <int NT, bool SHORT>
+  __device__ __forceinline__ void load_row(const Gram<NT, SHORT>& gr, const float* __restrict__ gb, int n,
+                                           int t) {
 #pragma unroll
-    for (int i = 0; i < 4; ++i) g[i] = *reinterpret_cast<const f32x4*>(p + 4 * i);
+    for (int i = 0; i < 4; ++i) {
+      if constexpr (SHORT)
+        g[i] = *reinterpret_cast<const f32x4*>(&gr.g[n][t][4 * i]);
+      else
+        g[i] = *reinterpret_cast<const f32x4*>(gb + (static_cast<size_t>(n) * C + t) * C + 4 * i);
+    }
   }
   // Row t for the solve. The entry it has no use for (15 forward, 0 backward) is kept alive to
   // here: a loaded register that nothing reads is reused, and waited for, right after its load.
@@ -416,26 +457,30 @@ struct StepIn {
   }
 };
 
-// Forward. TAPE: writes v - r and every chunk's entering state for the backward, else r.
-template <int NT, bool VEC, bool TAPE>
-__global__ void __launch_bounds__(NTH, 1) fwd_kernel(int T, int H, int nchunk,
-                                                     const float* __restrict__ k,
-                                                     const float* __restrict__ v,
-                                                     const float* __restrict__ beta,
-                                                     const float* __restrict__ gram,
-                                                     float* __restrict__ out,
-                                                     float* __restrict__ states) {
+template <int NT>
+struct FwdLds {
+  float kl[2][C][Geo<NT>::LS];
+  float pb[4][RB][ES];
+  float eb[C][ES];
+};
+
+// Forward. TAPE: writes v - r and every chunk's entering state for the backward, else r. `gram`:
+// the batch row's G (unless SHORT).
+template <int NT, bool VEC, bool TAPE, bool SHORT>
+__device__ __forceinline__ void fwd_body(FwdLds<NT>& m_, const Gram<NT, SHORT>& gr, int T, int H,
+                                         int nchunk, const float* __restrict__ k, const float* __restrict__ v,
+                                         const float* __restrict__ beta,
+                                         const float* __restrict__ gb, float* out, float* states) {
   using Ge = Geo<NT>;
-  __shared__ __attribute__((aligned(16))) float kl[2][C][Ge::LS];
-  __shared__ __attribute__((aligned(16))) float pb[4][RB][ES];
-  __shared__ __attribute__((aligned(16))) float eb[C][ES];
+  auto& kl = m_.kl;
+  auto& pb = m_.pb;
+  auto& eb = m_.eb;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int rb = blockIdx.x, b = blockIdx.y;
   const int c0 = wave * 16 * NT;
   const int t = lane & 15, lr = 4 * wave + (lane >> 4), row = rb * RB + lr;
   const size_t base = static_cast<size_t>(b) * T * H;
   const float* kb = k + base;
-  const float* gb = gram + static_cast<size_t>(b) * nchunk * C * C + t * C;
   f32x4 s[NT];
 #pragma unroll
   for (int n = 0; n < NT; ++n) s[n] = (f32x4){0.f, 0.f, 0.f, 0.f};
@@ -445,7 +490,7 @@ __global__ void __launch_bounds__(NTH, 1) fwd_kernel(int T, int H, int nchunk,
     q.x = v[base + static_cast<size_t>(tt) * H + min(row, H - 1)];
     q.beta = beta[static_cast<size_t>(b) * T + tt];
     q.f = 0.0f;
-    q.load_row(gb + static_cast<size_t>(n) * C * C);
+    q.load_row(gr, gb, n, t);
     return q;
   };
   Stage<NT, VEC> st;
@@ -497,33 +542,54 @@ __global__ void __launch_bounds__(NTH, 1) fwd_kernel(int T, int H, int nchunk,
   }
 }
 
-// Backward, chunks from the last. dk goes out as one partial per row block ([B][T][nrb][H]),
-// dbeta as one value per row block ([B][T][nrb]); reduce_kernel adds them in order.
-template <int NT, bool VEC>
+template <int NT, bool VEC, bool SHORT>
+__global__ void __launch_bounds__(NTH, 1) fwd_kernel(int T, int H, int nchunk,
+                                                     const float* __restrict__ k,
+                                                     const float* __restrict__ v,
+                                                     const float* __restrict__ beta,
+                                                     const float* __restrict__ gram,
+                                                     float* __restrict__ out) {
+  __shared__ __attribute__((aligned(16))) FwdLds<NT> m;
+  __shared__ __attribute__((aligned(16))) Gram<NT, SHORT> gr;
+  gr.template fill<VEC>(k + static_cast<size_t>(blockIdx.y) * T * H, T, H, nchunk);
+  fwd_body<NT, VEC, false, SHORT>(m, gr, T, H, nchunk, k, v, beta,
+                           gram + static_cast<size_t>(blockIdx.y) * nchunk * C * C, out, nullptr);
+}
+
+// Backward: the forward again for v - r and the entering states, which only this workgroup
+// reads, then the chunks from the last. dk goes out as one partial per row block
+// ([B][T][nrb][H]), dbeta as one value per row block ([B][T][nrb]); reduce_kernel adds them in
+// order.
+template <int NT, bool VEC, bool SHORT>
 __global__ void __launch_bounds__(NTH, 1) bwd_kernel(int T, int H, int nchunk,
                                                      const float* __restrict__ k,
-                                                     const float* __restrict__ ftape,
+                                                     const float* __restrict__ v,
                                                      const float* __restrict__ beta,
                                                      const float* __restrict__ g,
                                                      const float* __restrict__ gram,
-                                                     const float* __restrict__ states,
+                                                     float* ftape, float* states,
                                                      float* __restrict__ dv,
                                                      float* __restrict__ pdk,
                                                      float* __restrict__ pbeta) {
   using Ge = Geo<NT>;
-  __shared__ __attribute__((aligned(16))) float kl[2][C][Ge::LS];
+  __shared__ __attribute__((aligned(16))) FwdLds<NT> m_;
+  __shared__ __attribute__((aligned(16))) Gram<NT, SHORT> gr;
   __shared__ __attribute__((aligned(16))) float at[RB][Ge::LS];  // A_end as [row][column]
-  __shared__ __attribute__((aligned(16))) float pb[4][RB][ES];
   __shared__ __attribute__((aligned(16))) float db[C][ES];
-  __shared__ __attribute__((aligned(16))) float eb[C][ES];
   __shared__ float bb[C][ES];
+  auto& kl = m_.kl;
+  auto& pb = m_.pb;
+  auto& eb = m_.eb;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int rb = blockIdx.x, b = blockIdx.y, nrb = gridDim.x;
   const int c0 = wave * 16 * NT, hi = 4 * (lane >> 4), lo = lane & 15;
   const int t = lo, lr = 4 * wave + (lane >> 4), row = rb * RB + lr;
   const size_t base = static_cast<size_t>(b) * T * H;
   const float* kb = k + base;
-  const float* gb = gram + static_cast<size_t>(b) * nchunk * C * C + t * C;
+  const float* gb = gram + static_cast<size_t>(b) * nchunk * C * C;
+  gr.template fill<VEC>(kb, T, H, nchunk);
+  fwd_body<NT, VEC, true, SHORT>(m_, gr, T, H, nchunk, k, v, beta, gb, ftape, states);
+  __syncthreads();  // the tape and the states are read by other threads than wrote them
   f32x4 a[NT];
 #pragma unroll
   for (int n = 0; n < NT; ++n) a[n] = (f32x4){0.f, 0.f, 0.f, 0.f};
@@ -534,7 +600,7 @@ __global__ void __launch_bounds__(NTH, 1) bwd_kernel(int T, int H, int nchunk,
     q.x = g[o];
     q.f = ftape[o];
     q.beta = beta[static_cast<size_t>(b) * T + tt];
-    q.load_row(gb + static_cast<size_t>(n) * C * C);
+    q.load_row(gr, gb, n, t);
     return q;
   };
   Stage<NT, VEC> st;
@@ -671,7 +737,7 @@ static Layout layout(int64_t B, int64_t T, int64_t H, bool backward) {
   const size_t bt = static_cast<size_t>(B) * T;
   auto up = [](size_t x) { return (x + 255) & ~static_cast<size_t>(255); };
   Layout l{};
-  size_t o = up(static_cast<size_t>(B) * nchunk * C * C * 4);
+  size_t o = brief(B, T, H) ? 0 : up(static_cast<size_t>(B) * nchunk * C * C * 4);
   if (backward) {
     l.ftape = o; o = up(o + bt * H * 4);
     l.states = o; o = up(o + static_cast<size_t>(B) * nrb * nchunk * RB * 64 * tiles_for(H) * 4);
@@ -683,30 +749,30 @@ static Layout layout(int64_t B, int64_t T, int64_t H, bool backward) {
 }
 
 // Forward (out = r), or backward (g given).
-template <int NT, bool VEC>
+template <int NT, bool VEC, bool SHORT>
 static void launch(int64_t B, int64_t T, int64_t H, const float* k, const float* v,
                    const float* beta, const float* g, float* out, float* dk, float* dv,
                    float* dbeta, uint8_t* ws, hipStream_t stream) {
   const Layout l = layout(B, T, H, g != nullptr);
   const int nchunk = static_cast<int>((T + C - 1) / C), nrb = static_cast<int>((H + RB - 1) / RB);
   float* gram = reinterpret_cast<float*>(ws + l.gram);
-  const int64_t total = B * nchunk;
-  hipLaunchKernelGGL((gram_kernel<VEC>), dim3(static_cast<unsigned>((total + 3) / 4)), dim3(NTH), 0,
-                     stream, (int)T, (int)H, nchunk, total, k, gram);
+  if constexpr (!SHORT) {
+    const int64_t total = B * nchunk;
+    hipLaunchKernelGGL((gram_kernel<VEC>), dim3(static_cast<unsigned>((total + 3) / 4)), dim3(NTH), 0,
+                       stream, (int)T, (int)H, nchunk, total, k, gram);
+  }
   const dim3 grid(static_cast<unsigned>(nrb), static_cast<unsigned>(B));
   if (!g) {
-    hipLaunchKernelGGL((fwd_kernel<NT, VEC, false>), grid, dim3(NTH), 0, stream, (int)T, (int)H,
-                       nchunk, k, v, beta, gram, out, nullptr);
+    hipLaunchKernelGGL((fwd_kernel<NT, VEC, SHORT>), grid, dim3(NTH), 0, stream, (int)T, (int)H, nchunk,
+                       k, v, beta, gram, out);
     return;
   }
   float* ftape = reinterpret_cast<float*>(ws + l.ftape);
   float* states = reinterpret_cast<float*>(ws + l.states);
   float* pdk = reinterpret_cast<float*>(ws + l.pdk);
   float* pbeta = reinterpret_cast<float*>(ws + l.pbeta);
-  hipLaunchKernelGGL((fwd_kernel<NT, VEC, true>), grid, dim3(NTH), 0, stream, (int)T, (int)H, nchunk,
-                     k, v, beta, gram, ftape, states);
-  hipLaunchKernelGGL((bwd_kernel<NT, VEC>), grid, dim3(NTH), 0, stream, (int)T, (int)H, nchunk, k,
-                     ftape, beta, g, gram, states, dv, pdk, pbeta);
+  hipLaunchKernelGGL((bwd_kernel<NT, VEC, SHORT>), grid, dim3(NTH), 0, stream, (int)T, (int)H, nchunk, k,
+                     v, beta, g, gram, ftape, states, dv, pdk, pbeta);
   const int64_t BT = B * T;
   hipLaunchKernelGGL(reduce_kernel, dim3(static_cast<unsigned>((BT * H + NTH - 1) / NTH)), dim3(NTH),
                      0, stream, BT, (int)H, nrb, pdk, pbeta, dk, dbeta);
@@ -716,16 +782,27 @@ static int run(int64_t B, int64_t T, int64_t H, const float* k, const float* v, 
                const float* g, float* out, float* dk, float* dv, float* dbeta, uint8_t* ws,
                hipStream_t stream) {
   const bool vec = H % 4 == 0 && (reinterpret_cast<uintptr_t>(k) & 15u) == 0;
+  const bool in_lds = brief(B, T, H);
   switch (tiles_for(H)) {
-#define DABSN_CASE(N)                                                                       \
-  case N:                                                                                   \
-    if (vec)                                                                                \
-      launch<N, true>(B, T, H, k, v, beta, g, out, dk, dv, dbeta, ws, stream);              \
-    else                                                                                    \
-      launch<N, false>(B, T, H, k, v, beta, g, out, dk, dv, dbeta, ws, stream);             \
+#define DABSN_RUN(N, SHORT)                                                                   \
+  if (vec)                                                                                    \
+    launch<N, true, SHORT>(B, T, H, k, v, beta, g, out, dk, dv, dbeta, ws, stream);           \
+  else                                                                                        \
+    launch<N, false, SHORT>(B, T, H, k, v, beta, g, out, dk, dv, dbeta, ws, stream)
+#define DABSN_CASE(N)      \
+  case N:                  \
+    if (in_lds) {          \
+      DABSN_RUN(N, true);  \
+    } else {               \
+      DABSN_RUN(N, false); \
+    }                      \
     break;
-    DABSN_CASE(1) DABSN_CASE(2) DABSN_CASE(4) DABSN_CASE(8)
+    DABSN_CASE(1) DABSN_CASE(2) DABSN_CASE(4)
 #undef DABSN_CASE
+    case 8:
+      DABSN_RUN(8, false);
+      break;
+#undef DABSN_RUN
   }
   DABSN_HIP_CHECK(hipGetLastError());
   return DABSN_OK;
@@ -770,8 +847,8 @@ int dabsn_hip_permanent_scan_fwd_ws(int64_t B, int64_t T, int64_t H, const float
     return dabsn_hip_permanent_scan_fwd(B, T, H, key, value, beta, out, stream);
   DABSN_REQUIRE(out, "permanent scan: null output");
   if (T == 0) return DABSN_OK;
-  const size_t need = chunked::layout(B, T, H, false).end;
-  DABSN_REQUIRE(workspace && workspace_bytes >= need, "permanent scan: workspace %zu < %zu",
+  const size_t need = chunked::layout(B, T, H, false).end;  // none for short scans
+  DABSN_REQUIRE(need == 0 || (workspace && workspace_bytes >= need), "permanent scan: workspace %zu < %zu",
                 workspace_bytes, need);
   return chunked::run(B, T, H, key, value, beta, nullptr, out, nullptr, nullptr, nullptr,
                       static_cast<uint8_t*>(workspace), stream);

@@ -650,7 +650,7 @@ def permanent_delta_scan(k: Tensor, v: Tensor, beta: Tensor) -> Tensor:
     kf, vf, bf = (x.float().contiguous() for x in (k, v, beta))
     out = torch.empty((B, T, H), device=k.device, dtype=torch.float32)
     nbytes = lib.dabsn_hip_permanent_scan_fwd_workspace_bytes(B, T, H)
-    ws = torch.empty(max(nbytes, 4), dtype=torch.uint8, device=k.device)
+    ws = torch.empty(nbytes, dtype=torch.uint8, device=k.device) if nbytes else None
     tk = KernelTimer.begin("permanent_scan_fwd", k)
     _lib.check(lib.dabsn_hip_permanent_scan_fwd_ws(B, T, H, _p(kf), _p(vf), _p(bf), _p(out),
                                                    _p(ws), nbytes, _stream(k)), "permanent scan")

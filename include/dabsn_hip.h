@@ -619,7 +619,8 @@ int dabsn_hip_permanent_scan_fwd(int64_t B, int64_t T, int64_t H, const float* k
                                  hipStream_t stream);
 /* The same scan in chunks of 16 steps as fp32 matrix products (H <= 512; wider states walk
  * step by step as above), with a workspace of
- * dabsn_hip_permanent_scan_fwd_workspace_bytes() for the chunks' key products. */
+ * dabsn_hip_permanent_scan_fwd_workspace_bytes() for the chunks' key products (0 for short
+ * scans, which keep them in LDS; the workspace may then be NULL). */
 size_t dabsn_hip_permanent_scan_fwd_workspace_bytes(int64_t B, int64_t T, int64_t H);
 int dabsn_hip_permanent_scan_fwd_ws(int64_t B, int64_t T, int64_t H, const float* key,
                                     const float* value, const float* beta, float* out,

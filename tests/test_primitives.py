@@ -111,6 +111,44 @@ def test_permanent_scan_chunk_and_tile_edges(cuda_device, B, T, H):
         assert float(err) <= 1e-5 * max(float(w.norm()), 1e-30)
 
 
+def test_short_permanent_scans_need_no_forward_workspace():
+    from dabsn_amd import _lib
+
+    size = _lib.load().dabsn_hip_permanent_scan_fwd_workspace_bytes
+    for H, longest in ((1, 128), (128, 128), (129, 64), (256, 64)):
+        assert size(3, 1, H) == size(3, longest, H) == 0 < size(3, longest + 1, H)
+    assert size(3, 1, 257) > 0 and size(3, 129, 513) == 0
+    assert size(256, 64, 128) == 0 < size(257, 64, 128)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("B,T,H", [(2, 112, 33), (1, 113, 128), (2, 127, 100), (1, 128, 129),
+                                   (1, 128, 128), (2, 129, 64), (1, 64, 256), (1, 65, 256), (1, 64, 257),
+                                   (3, 63, 251), (3, 145, 20)])
+def test_permanent_scan_short_scan_edges(cuda_device, B, T, H):
+    """Up to 128 steps at H <= 128 and 64 at H <= 256 a workgroup forms the chunks' key products itself,
+    beyond they come from a kernel of their own: forward and backward against fp64, 1e-5 in
+    the norm as above."""
+    test_permanent_scan_chunk_and_tile_edges(cuda_device, B, T, H)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("T", [1, 37, 150])
+@pytest.mark.parametrize("H", [1, 64, 65, 200, 512])
+def test_permanent_scan_entry_without_workspace(cuda_device, H, T):
+    """The C entry that takes no workspace walks step by step at every width: the operator's
+    values in another order of summation, 1e-5 in the norm."""
+    from dabsn_amd import _lib
+
+    k, v, beta, _ = (x.to(cuda_device) for x in _permanent_case(H + T, 2, T, H))
+    out = torch.full_like(v, float("nan"))
+    p = lambda t: t.data_ptr()  # noqa: E731
+    assert _lib.load().dabsn_hip_permanent_scan_fwd(2, T, H, p(k), p(v), p(beta), p(out),
+                                                    ops._stream(k)) == 0
+    want = ops.permanent_delta_scan(k, v, beta)
+    assert float((out - want).norm()) <= 1e-5 * max(float(want.norm()), 1e-30)
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("H", [40, 200])
 def test_permanent_scan_keeps_a_bad_step_out_of_the_steps_before_it(cuda_device, H):
