@@ -398,6 +398,29 @@ def test_long_scan_block_edges(cuda_device, dtype, B, T, H):
     assert torch.equal(got[:, :, keep], out[0][:, :, keep])
 
 
+@pytest.mark.parametrize("dtype,T,H", [(torch.bfloat16, 70, (1 << 24) + 1), (torch.float32, 33, 1 << 24)])
+def test_long_scan_rows_past_32_bit_offsets(cuda_device, dtype, T, H):
+    """2^24 channels and more take plain 64-bit addresses: spans of the channels are those of
+    calls on the spans alone, bit for bit (channels are independent), forward, backward and
+    accumulating backward."""
+    g = torch.Generator(device=cuda_device).manual_seed(T)
+    r = lambda *s: torch.randn(*s, device=cuda_device, dtype=dtype, generator=g)  # noqa: E731
+    f = lambda *s: torch.randn(*s, device=cuda_device, generator=g)  # noqa: E731
+    w, p, go = r(1, T, H), r(1, T, H).sigmoid_(), r(1, T, H)
+    lg = [torch.tensor([v], device=cuda_device) for v in (2.2, 2.0, 2.4, 1.4)]
+    st, gf = [f(1, H) for _ in range(3)], [f(1, H) for _ in range(3)]
+    out = ops.long_scan_window(w, p, lg, *st)
+    res = ops.long_scan_backward_parts(w, p, lg, out[4], go, *gf)
+    acc = ops.long_scan_backward_parts(w, p, lg, out[4], go, *gf, go.clone(), torch.empty_like(go))
+    for s in (slice(0, 100), slice(H // 2 - 50, H // 2 + 50), slice(H - 100, H)):
+        c = lambda x: x[..., s].contiguous()  # noqa: E731
+        o = ops.long_scan_window(c(w), c(p), lg, *map(c, st))
+        b = ops.long_scan_backward_parts(c(w), c(p), lg, o[4], c(go), *map(c, gf))
+        assert all(torch.equal(c(x), y) for x, y in zip(out, o))
+        assert all(torch.equal(c(x), y) for x, y in zip((*res[:2], *res[3]), (*b[:2], *b[3])))
+        assert torch.equal(c(acc[0]), c(go) + b[0]) and torch.equal(c(acc[1]), b[1])
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("B,T,H", [(2, 127, 70), (2, 128, 70), (64, 128, 64), (65, 128, 64)])
 def test_long_scan_backward_accumulates_with_and_without_workspace(cuda_device, dtype, B, T, H):

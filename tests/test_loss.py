@@ -174,6 +174,34 @@ def test_split_gradient_planes_hold_the_fp32_gradient(cuda_device, rows, V):
 
 
 @pytest.mark.gpu
+def test_split_gradient_planes_below_their_exact_range(cuda_device):
+    """Gradients of words whose logits lie up to 100 below the largest: the planes hold every
+    bit of a value of at least 2^-110 and all but what lies below bf16's smallest subnormal,
+    2^-133, of a smaller one."""
+    from dabsn_amd import _lib
+    from dabsn_amd.kernels import ops
+
+    rows, V = 5, 808
+    x = (-torch.arange(V, dtype=torch.float32) / 8).repeat(rows, 1)
+    x = x.to(torch.bfloat16).to(cuda_device)
+    t = torch.zeros(rows, dtype=torch.int64, device=cuda_device)
+    lse, _ = ops.ce_rows(x, t, -100)
+    scale = torch.tensor([0.37], device=cuda_device)
+    want = ops.ce_rows_backward(x, t, -100, lse, scale).double()
+    lib = _lib.load()
+    planes = torch.zeros(3, rows, V, device=cuda_device, dtype=torch.bfloat16)
+    word = torch.zeros(1, device=cuda_device, dtype=torch.int32)
+    p = lambda v: v.data_ptr()  # noqa: E731
+    assert lib.dabsn_hip_ce_split(rows, V, p(x), V, p(t), -100, p(lse), p(scale), p(planes),
+                                  rows * V, V, None, p(word), None) == 0
+    torch.cuda.synchronize()
+    err = (planes.double().sum(0) - want).abs()
+    exact = want.abs() >= 2.0 ** -110
+    assert bool(exact.any()) and bool((~exact & (want != 0)).any())
+    assert float(err[exact].max()) == 0 and float(err.max()) <= 2.0 ** -133
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("N,V,H,budget,bias", [(1, 5, 3, None, True), (70, 33, 48, 16 * 33, True),
                                                (64, 129, 96, 16 * 129, False),
                                                (300, 1000, 200, 40 * 1000, True),
