@@ -114,9 +114,10 @@ struct Logits {
 };
 
 // tanh(y) for y >= 0 without a branch (the library's takes one per range, both in a wave whose
-// lanes disagree, and the unrolled steps around it cannot be interleaved). Below 0.625 the odd
-// polynomial y + y^3 q(y^2), q fitted to (tanh y - y) / y^3 by minimax least squares (relative
-// error 4.4e-9, and 8.5e-9 with the coefficients rounded to fp32); above, 1 - 2 / (exp(2y) + 1). At most 2 ulp, on average 2.4e-8
+// lanes disagree, and the unrolled steps around it cannot be interleaved). The range is split
+// as in the Cephes library's tanhf. Below 0.625 the odd polynomial y + y^3 q(y^2), q fitted to
+// (tanh y - y) / y^3 by minimax least squares (relative error 4.4e-9, and 8.5e-9 with the
+// coefficients rounded to fp32); above, 1 - 2 / (exp(2y) + 1). At most 2 ulp, on average 2.4e-8
 // relative. NaN stays NaN, infinity gives 1.
 __device__ __forceinline__ float tanh_abs(float y) {
   const float z = y * y;

@@ -151,8 +151,9 @@ __device__ __forceinline__ void split3(float v, bf16 (&o)[3]) {
   o[2] = static_cast<bf16>(__builtin_bit_cast(uint32_t, r2) >> 16);
 }
 
-// Bound by memory: 2 bytes read and 6 written per element (29.5 us for 524 rows of 32,000,
-// 4.5 TB/s; the fp32 gradient took 21.8 us plus 41 us for its column sums). A block owns kSplitRows rows of a strip of columns: a row's target, logsumexp
+// Bound by memory: 2 bytes read and 6 written per element (31 us for 524 rows of 32,000, the
+// average of a kernel trace: 4.3 TB/s; the fp32 gradient took 21.8 us plus 41 us for its
+// column sums). A block owns kSplitRows rows of a strip of columns: a row's target, logsumexp
 // and validity are uniform, and each thread carries its columns' sums over the rows (the
 // bias gradient's partials, one row of `part` per block row), which the fp32 gradient took
 // another pass over memory for.

@@ -283,8 +283,10 @@ class DABSNRead(nn.Module):
         if members is None:
             admission = glue.admission_for_select()
             # The successor fold serves every read of gathered rows: one product with V in
-            # place of two (V and the successor rows). B=32, T=3200, H=256 fp32 without
-            # autograd: 4622 us without the fold, 3395 with it.
+            # place of two (V and the successor rows) where every slot's successor is a bank
+            # row. B=32, T=3200, H=256 fp32 without autograd, every position admitted: 4622
+            # us without the fold, 3395 with it; 1,803 of them, scattered (two products
+            # either way): 3248 without asking for the fold, 3128 with it.
             want_fold = gathers and admission.is_cuda
             n_max, idx, valid, next_idx, rank, fold, read_idx = self._select(
                 admission, length, width, want_fold, query_start)

@@ -667,8 +667,9 @@ int dabsn_hip_ce_bwd(int dtype, int64_t rows, int64_t V, const void* logits, int
                      const float* scale, float* dlogits, uint32_t* err, hipStream_t stream);
 /* The backward of bf16 logits as three bf16 planes whose sum is the fp32 gradient, bit for
  * bit from 2^-110 up and to 2^-133 below (planes + k * plane, row stride ldp >= V, k = 0..2):
- * the gradient products then run as bf16 matrix products. part (NULL or [dabsn_hip_ce_split_parts(rows)][V]) receives partial
- * column sums of the fp32 gradient; dabsn_hip_ce_bias sums them in order into gbias [V] (added
+ * the gradient products then run as bf16 matrix products. part (NULL or
+ * [dabsn_hip_ce_split_parts(rows)][V]) receives partial column sums of the fp32 gradient;
+ * dabsn_hip_ce_bias sums them in order into gbias [V] (added
  * to it with `add`). dabsn_hip_ce_join: out (bf16 [n]) = the sum of three fp32 [n] arrays. */
 int64_t dabsn_hip_ce_split_parts(int64_t rows);
 int dabsn_hip_ce_split(int64_t rows, int64_t V, const void* logits, int64_t ldl,
